@@ -15,35 +15,48 @@
 // compute it: eight fused multiply-add chains (chain L takes dims L, L + 8,
 // ... in order), combined ((s0+s4)+(s1+s5)) + ((s2+s6)+(s3+s7)), times
 // 1/(sqrt(dim) p), times the key's scale; the query rotation repeats the
-// reference's float steps (attention.cpp:528-550, fwht.cpp:33-66).  A lane
-// owns one token of a 64-token tile with its dequantised K row in registers,
-// and the rotated query entries, uniform across the wave, come from the
-// scalar cache as the FMAs' SGPR operand: the FMA stream has no other
-// operand traffic.  The V sum runs on v_mfma_f32_16x16x4f32, the softmax
-// weight and the V scale folded into its A operand (fp32 accumulation, as the
-// reference's).  The online softmax is the LUT kernel's with the reference's
-// -1e30 seed, in natural units (exp2 of (logit - max) * log2 e, so the
-// weights of the tokens near the maximum carry no rounding of the logit's
-// magnitude); splits over tokens end in decode.hip's finalize kernel.
+// reference's float steps (attention.cpp:528-550, fwht.cpp:33-66).
 //
-// Operand layouts (established on the device): lane l supplies A[l % 16][l /
-// 16] and B[l / 16][l % 16]; result register r of lane l is D[4 (l / 16) +
-// r][l % 16].  The V product takes queries as M and tokens as K, so lane l
-// supplies the weight of query l % 16 and token 4 r + l / 16 of each 16-token
-// subtile at k-step r; the logits (one token per lane) reach that layout
-// through LDS.
+// Both products run on the matrix cores.  v_mfma_f32_16x16x4 adds its four
+// products to an entry one after another, in order, each a fused multiply-add
+// rounded as fmaf (checked on the device against fmaf, bit for bit, over
+// normal, denormal and large operands), so a chain of it is a chain of the
+// reference's: eight accumulators, chain L of a 16-token by 16-query tile fed
+// dims L + 8 j, j ascending, four an instruction.  Operand layouts
+// (established on the device): lane l supplies A[l % 16][l / 16] and
+// B[l / 16][l % 16], register r of lane l is D[4 (l / 16) + r][l % 16].  Keys
+// are A and queries B, so a lane holds all eight chain sums of its tokens and
+// query, and combines them without leaving its registers.  The V sum takes
+// queries as M and, at step r, tokens 4 k + r as K: A is the weight that the
+// lane already has from the logits.  The softmax weight and
+// the V scale are folded into A (fp32 accumulation, as the reference's).  The
+// online softmax is the LUT kernel's with the reference's -1e30 seed, in
+// natural units (exp2 of (logit - max) * log2 e, so the weights of the tokens
+// near the maximum carry no rounding of the logit's magnitude); splits over
+// tokens end in decode.hip's finalize kernel.
 //
-// Block: kMqWaves (8) waves and kMqQueries (16) queries of one head over one
-// token split.  Every wave handles all 16 queries; the waves split the
-// tokens: wave w takes the 64-token tiles starting at t_begin + 64 w, then
-// every 64 kMqWaves tokens.  Lane l owns token l of its wave's tile: the K
-// row, dequantised through the codebook in LDS into registers (the next
-// tile's row requested a tile ahead; rows stored in XOR byte order,
-// device.hpp kperm_mask, are read back in reference order by load_k_row),
-// and the V slices the MFMA's B operand takes from global memory.  A wave's
-// logits reach the MFMA layout through its own LDS region (transposed, row
-// stride 17); at the end the waves' (m, l, acc) records meet in LDS and are
-// merged per query.
+// Block: four waves, QG (1, 2 or 4) groups of 16 queries of one head, one
+// token split.  The block takes TS = 4 / QG tiles of 16 tokens a step: its
+// threads turn the tiles' codes into floats in LDS, a unit of 8 dims each
+// (16-entry tables, distinct banks), one step ahead of their use; wave (slice
+// ts, group) multiplies tile ts with its group's queries.  Lane (g, c) =
+// (l / 16, l % 16) holds, for query c, the rotated entries of the 8-dim groups
+// 4 i + g in registers; reads the same groups of token c's key (16-byte LDS
+// reads, a step of four chains each) and, for tokens 4 g + r, the value's dims
+// 4 c .. 4 c + 3 and 64 + 4 c .. (likewise).  Rows are padded so that 16
+// lanes' reads cover the 64 banks.  Slices of the same queries merge in LDS at
+// the end.
+//
+// Bound: the matrix cores' fp32 rate, and the vector ALU's work beside it
+// (about 180 instructions a tile and wave, which the fp32 matrix rate does not
+// hide: taking either product out shortens the launch by exactly its own 26
+// us).  64 queries of 8 heads over 32,768 tokens at padded 128, K4/V4 (8.6
+// GFLOP, 55 us at 157 TFLOP/s): 102 us under the profiler.  The kernel before
+// it ran the logits' chains on the vector ALU, a token a lane, and passed them
+// to the V product through LDS: 156 us.  With a wave dequantising its own
+// tiles (codes read by the four lanes of a token, tables to registers) the
+// matrix form took 175 us: sixteen code loads and 128 table reads a tile and
+// wave, and 20 registers spilled.
 #include <algorithm>
 
 #include "launch.hpp"
@@ -54,93 +67,79 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kMqWaves = 8;
+constexpr int kMqWaves = 4;
 constexpr int kMqThreads = 64 * kMqWaves;
-constexpr int kMqQueries = 16;  // queries per block, shared by its waves
-constexpr int kMqTile = 64;     // tokens per wave step (one per lane)
+constexpr int kMqQueries = 16;  // queries per wave
+constexpr int kMqTile = 16;     // tokens per wave step
 constexpr float kLog2e = 1.44269504088896340736f;
 
-// Code k (MSB-first packing, quantizer.cpp:156-209) of a little-endian word
-// stream w[] holding a row's bytes from byte 0.
+// The codes of dims 8 j .. 8 j + 7 of a packed row (MSB-first,
+// quantizer.cpp:156-209), as loaded: 4 bits a word, 2 bits a half word, 3 bits
+// the two words that hold the 24-bit big-endian group (the second clamped to
+// the row).  K rows of 2/4-bit codes are stored XOR-permuted (device.hpp
+// kperm_mask; x = slot & mask, 0 for V): the unit's bytes sit at unit j ^ (x /
+// unit bytes), permuted among themselves by x % unit bytes.
 template <int B>
-__device__ __forceinline__ uint32_t code_in(const uint32_t *w, int k) {
+struct MqUnit {
+  uint32_t w[B == 3 ? 2 : 1];
+};
+
+template <int P, int B>
+__device__ __forceinline__ MqUnit<B> mq_load_unit(const uint8_t *codes, uint32_t slot, int j,
+                                                  uint32_t x) {
+  const uint8_t *row = codes + (size_t)slot * (P * B / 8);
+  MqUnit<B> u;
   if constexpr (B == 4) {
-    const int byte = k >> 1;
-    return (w[byte >> 2] >> (8 * (byte & 3) + ((k & 1) ? 0 : 4))) & 15u;
+    u.w[0] = reinterpret_cast<const uint32_t *>(row)[(uint32_t)j ^ (x >> 2)];
   } else if constexpr (B == 2) {
-    const int byte = k >> 2;
-    return (w[byte >> 2] >> (8 * (byte & 3) + 6 - 2 * (k & 3))) & 3u;
+    u.w[0] = reinterpret_cast<const uint16_t *>(row)[(uint32_t)j ^ (x >> 1)];
   } else {
-    // 3 bits: group G = k / 8 is the big-endian 24-bit value of bytes 3G..3G+2
-    const int G = k >> 3, b0 = 3 * G;
-    auto byte_at = [&](int b) { return (w[b >> 2] >> (8 * (b & 3))) & 0xFFu; };
-    const uint32_t v = (byte_at(b0) << 16) | (byte_at(b0 + 1) << 8) | byte_at(b0 + 2);
-    return (v >> (21 - 3 * (k & 7))) & 7u;
+    const uint32_t *r32 = reinterpret_cast<const uint32_t *>(row);
+    const int w0 = 3 * j / 4;
+    u.w[0] = r32[w0];
+    u.w[1] = r32[min(w0 + 1, P * 3 / 32 - 1)];
+  }
+  return u;
+}
+
+// The unit's eight values.
+template <int B>
+__device__ __forceinline__ void mq_unit_values(const MqUnit<B> &u, int j, uint32_t x,
+                                               const float *s_cb, float (&v)[8]) {
+  if constexpr (B == 4) {
+    const uint32_t w = __builtin_amdgcn_perm(0u, u.w[0], 0x03020100u ^ ((x & 3u) * 0x01010101u));
+#pragma unroll
+    for (int d = 0; d < 8; ++d) v[d] = s_cb[(w >> (8 * (d >> 1) + ((d & 1) ? 0 : 4))) & 15u];
+  } else if constexpr (B == 2) {
+    const uint32_t w = __builtin_amdgcn_perm(0u, u.w[0], 0x0C0C0100u ^ ((x & 1u) * 0x0101u));
+#pragma unroll
+    for (int d = 0; d < 8; ++d) v[d] = s_cb[(w >> (8 * (d >> 2) + 6 - 2 * (d & 3))) & 3u];
+  } else {
+    // bytes 3 j .. 3 j + 2, from byte (3 j) % 4 of the word pair, big-endian
+    const uint32_t a = __builtin_amdgcn_alignbyte(u.w[1], u.w[0], (uint32_t)(3 * j) & 3u);
+    const uint32_t w = __builtin_amdgcn_perm(0u, a, 0x0C000102u);
+#pragma unroll
+    for (int d = 0; d < 8; ++d) v[d] = s_cb[(w >> (21 - 3 * d)) & 7u];
   }
 }
 
-// The K row of `slot` in reference byte order, as little-endian words.  Rows
-// of 2/4-bit codes are stored XOR-permuted (device.hpp kperm_mask): reference
-// word w sits at stored word w ^ (x >> 2) with its bytes permuted by x & 3,
-// x = slot & mask.
-template <int P, int KB>
-__device__ __forceinline__ void load_k_row(const HeadDesc *d, uint32_t slot, uint32_t *kw) {
-  constexpr int W = P * KB / 32;
-  const uint32_t *r32 = reinterpret_cast<const uint32_t *>(d->k_codes + (size_t)slot * (P * KB / 8));
-  if constexpr (KB == 3) {
-#pragma unroll
-    for (int i = 0; i < W; ++i) kw[i] = r32[i];
-  } else {
-    constexpr uint32_t xmask = (uint32_t)kperm_mask(P, KB);
-    const uint32_t x = slot & xmask;
-    const uint32_t sel = 0x03020100u ^ ((x & 3u) * 0x01010101u);
-    if constexpr (W % 4 == 0) {
-      // whole 16-byte chunks: chunk c of the reference row is stored chunk c ^ (x >> 4)
-      const uint4 *r128 = reinterpret_cast<const uint4 *>(r32);
-#pragma unroll
-      for (int c = 0; c < W / 4; ++c) {
-        const uint4 v = r128[c ^ (x >> 4)];
-        const uint32_t q[4] = {v.x, v.y, v.z, v.w};
-        const uint32_t xw = (x >> 2) & 3u;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          // reference word 4c + i is stored word (4c + i) ^ (x >> 2): in chunk c ^ (x >> 4), slot i ^ xw
-          uint32_t sw = q[0];
-          sw = xw == (uint32_t)(i ^ 1) ? q[1] : sw;
-          sw = xw == (uint32_t)(i ^ 2) ? q[2] : sw;
-          sw = xw == (uint32_t)(i ^ 3) ? q[3] : sw;
-          kw[4 * c + i] = __builtin_amdgcn_perm(0u, sw, sel);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < W; ++i) kw[i] = __builtin_amdgcn_perm(0u, r32[i ^ (x >> 2)], sel);
-    }
-  }
-}
-
-// This lane's V codes: the P / 16 codes of dims [P/16 c, P/16 (c + 1)) of
-// the row (V rows are unpermuted MSB-first bit streams), left-aligned in a
-// word, code i in bits [32 - VB (i + 1), 32 - VB i).
-template <int P, int VB>
-__device__ __forceinline__ uint32_t v_slice(const uint8_t *row, int c) {
-  constexpr int BITS = (P / 16) * VB, ROWW = P * VB / 32;
-  const uint32_t *r32 = reinterpret_cast<const uint32_t *>(row);
-  const int b0 = c * BITS;
-  const int w0 = b0 >> 5;
-  const uint32_t a = __builtin_bswap32(r32[w0]);
-  if constexpr (32 % BITS == 0) {
-    return a << (b0 & 31);  // the slice never straddles a word
-  } else {
-    const uint32_t b = __builtin_bswap32(r32[min(w0 + 1, ROWW - 1)]);
-    const uint64_t win = ((uint64_t)a << 32) | b;
-    return (uint32_t)((win << (b0 & 31)) >> 32);
-  }
+// max(v) over the four lanes that share lane % 16.
+__device__ __forceinline__ float quad_max(float v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
 // Read-only global memory seen through the constant address space: loads at
 // wave-uniform addresses become scalar loads.
 typedef const __attribute__((address_space(4))) float cfloat;
+// The descriptor read this way is uniform to the compiler too: loops over a
+// ring's tokens stay scalar branches, barriers inside them included.
+typedef const __attribute__((address_space(4))) HeadDesc cdesc;
+__device__ __forceinline__ cdesc *desc_of(HeadDesc *const *item_desc, int i) {
+  return (cdesc *)((const __attribute__((address_space(4))) uint64_t *)item_desc)[i];
+}
 
 // Rotated queries of query group qg of head h: rows of P floats at
 // qrot[((h * qgroups + qg) * 16 + jj) * P], zero rows past nq.  One wave per
@@ -213,171 +212,232 @@ __global__ __launch_bounds__(256) void mq_rotate_kernel(HeadDesc *const *item_de
 }
 
 
-// Block (split, head h, query group qg), 1-D grid with the split fastest:
-// the blocks resident together mostly share one head's 16 queries, 8 KB of
-// scalar-cache working set.  Wave w of the block takes the 64-token tiles w,
-// w + 4, ... of the block's token range on its own (no barriers in the token
-// loop) and the four waves' (m, l, acc) merge in LDS at the end.
-template <int P, int KB, int VB>
-__global__ __launch_bounds__(kMqThreads, 1) void decode_mq_kernel(
+// Block (split, head h, groups qg0 .. qg0 + QG - 1), 1-D grid with the split
+// fastest.
+template <int P, int KB, int VB, int QG>
+__global__ __launch_bounds__(kMqThreads, QG == 4 ? 3 : 2) void decode_mq_kernel(
     HeadDesc *const *item_desc, int n_heads, int nq, int qgroups, int chunk, int n_splits,
     const float *__restrict__ qrot, float *__restrict__ partials) {
-  constexpr int NT = P / 16;       // 16-column output tiles; lane c holds dims [NT c, NT c + NT)
-  constexpr int KW = P * KB / 32;  // words of a K row
-  constexpr int LST = 17;          // row stride of a wave's transposed logits
-  constexpr int MST = P + 4;       // row stride of a wave's merge record: m, l, pad, pad, acc
-  constexpr uint32_t vmask = (1u << VB) - 1u;
-  constexpr int SMEM = kMqWaves * kMqQueries * MST > kMqWaves * kMqTile * LST
-                           ? kMqWaves * kMqQueries * MST
-                           : kMqWaves * kMqTile * LST;
-  __shared__ __align__(16) float s_buf[SMEM];  // transposed logits; then the merge records
+  constexpr int TS = kMqWaves / QG;         // tiles a step
+  constexpr int NBUF = TS == 4 ? 1 : 2;     // LDS copies of a step's tiles
+  constexpr int NT = P / 16;                // 16-column output tiles
+  constexpr int NE = P / 4;                 // entries of a row a lane holds
+  constexpr int KST = NE + 4;               // K: [token][g][group 4 i + g], stride of a (token, g)
+  constexpr int VST = P + 4;                // V: [token][dim], stride of a token
+  constexpr int TILE = kMqTile * (4 * KST + VST) + 2 * kMqTile;  // K, V, both scales
+  constexpr int MST = P + 4;  // row stride of a wave's merge record: m, l, pad, pad, acc
+  constexpr int UNITS = TS * kMqTile * P / 8;  // units of K (and of V) a step
+  constexpr int UPT = (UNITS + kMqThreads - 1) / kMqThreads;
+  static_assert(UNITS % kMqThreads == 0 || UNITS < kMqThreads, "units spread evenly");
+  constexpr int SMEM = NBUF * TS * TILE;
+  static_assert(TS == 1 || SMEM >= kMqWaves * kMqQueries * MST, "the merge records fit");
+  __shared__ __align__(16) float s_buf[SMEM];
   __shared__ float s_cbk[16];
   __shared__ float s_cbv[16];
 
   const int bid = blockIdx.x;
   const int split = bid % n_splits, rest = bid / n_splits;
-  const int h = rest % n_heads, qg = rest / n_heads;
-  const HeadDesc *d = item_desc[h];
+  const int h = rest % n_heads, qg0 = (rest / n_heads) * QG;
+  cdesc *d = desc_of(item_desc, h);
   const int dim = d->dim, n = d->st.size;
   const int t_begin = split * chunk, t_end = min(n, t_begin + chunk);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c16 = lane & 15, g = lane >> 4;
-  const int j0 = qg * kMqQueries;  // first query of the block
+  const int ts = wave / QG, qg = qg0 + wave % QG;
+  const int j0 = qg * kMqQueries;  // first query of the wave
   auto part_of = [&](int j) {
     return partials + ((size_t)(j * n_heads + h) * n_splits + split) * (P + 4);
   };
 
   if (t_begin >= t_end) {
     // empty split: (m, l, acc) = (-inf, 0, 0) for the block's queries
-    for (int i = threadIdx.x; i < kMqQueries * (P + 4); i += kMqThreads) {
-      const int jj = i / (P + 4), e = i - jj * (P + 4);
-      if (j0 + jj < nq) part_of(j0 + jj)[e] = e == 0 ? -INFINITY : 0.0f;
+    for (int i = threadIdx.x; i < QG * kMqQueries * (P + 4); i += kMqThreads) {
+      const int jj = i / (P + 4), e = i - jj * (P + 4), j = qg0 * kMqQueries + jj;
+      if (j < nq) part_of(j)[e] = e == 0 ? -INFINITY : 0.0f;
     }
     return;
   }
 
-  if (threadIdx.x < (1 << KB)) s_cbk[threadIdx.x] = cb<KB>(threadIdx.x);
-  if (threadIdx.x < (1 << VB)) s_cbv[threadIdx.x] = cb<VB>(threadIdx.x);
-  __syncthreads();
-
-  // the block's 16 rotated queries (wave-uniform: scalar loads)
-  const cfloat *qw = (const cfloat *)(qrot + (size_t)(h * qgroups + qg) * kMqQueries * P);
   const float attn_s = 1.0f / (sqrtf((float)dim) * (float)P);
   const float isp = 1.0f / sqrtf((float)P);
-  const uint8_t *vbase = d->v_codes;
-  constexpr int v_pb = P * VB / 8;
-  float *s_lg = s_buf + wave * (kMqTile * LST);
+  const uint8_t *kbase = d->k_codes, *vbase = d->v_codes;
+  const float *k_scale = d->k_scale, *v_scale = d->v_scale;
+
+  // ---- a step's codes: units u = thread, thread + kMqThreads, ... of its TS
+  // tiles, unit (token u / (P / 8), dims 8 (u % (P / 8)) ..); tokens past the
+  // split's end are its last one (their weights are 0) ----
+  MqUnit<KB> ku[UPT];
+  MqUnit<VB> vu[UPT];
+  float sc = 0.0f;
+  const bool has_units = UNITS >= kMqThreads || (int)threadIdx.x < UNITS;
+  auto slot_of = [&](int t) { return (uint32_t)min(t, t_end - 1); };
+  auto load_step = [&](int tb) {
+    if (has_units) {
+#pragma unroll
+      for (int i = 0; i < UPT; ++i) {
+        const int u = (int)threadIdx.x + i * kMqThreads, tk = u / (P / 8), j = u % (P / 8);
+        const uint32_t slot = slot_of(tb + tk);
+        ku[i] = mq_load_unit<P, KB>(kbase, slot, j, slot & (uint32_t)kperm_mask(P, KB));
+        vu[i] = mq_load_unit<P, VB>(vbase, slot, j, 0u);
+      }
+    }
+    if (threadIdx.x < 2 * TS * kMqTile) {
+      const int tk = threadIdx.x % (TS * kMqTile);
+      sc = ((int)threadIdx.x < TS * kMqTile ? k_scale : v_scale)[slot_of(tb + tk)];
+    }
+  };
+  auto store_step = [&](int tb, float *buf) {
+    if (has_units) {
+#pragma unroll
+      for (int i = 0; i < UPT; ++i) {
+        const int u = (int)threadIdx.x + i * kMqThreads, tk = u / (P / 8), j = u % (P / 8);
+        float *tile = buf + (tk / kMqTile) * TILE;
+        const int t16 = tk % kMqTile;
+        const uint32_t x = slot_of(tb + tk) & (uint32_t)kperm_mask(P, KB);
+        float kv[8], vv[8];
+        mq_unit_values<KB>(ku[i], j, x, s_cbk, kv);
+        float4 *kr = reinterpret_cast<float4 *>(tile + (t16 * 4 + (j & 3)) * KST + 8 * (j >> 2));
+        kr[0] = make_float4(kv[0], kv[1], kv[2], kv[3]);
+        kr[1] = make_float4(kv[4], kv[5], kv[6], kv[7]);
+        mq_unit_values<VB>(vu[i], j, 0u, s_cbv, vv);
+        float4 *vr = reinterpret_cast<float4 *>(tile + kMqTile * 4 * KST + t16 * VST + 8 * j);
+        vr[0] = make_float4(vv[0], vv[1], vv[2], vv[3]);
+        vr[1] = make_float4(vv[4], vv[5], vv[6], vv[7]);
+      }
+    }
+    if (threadIdx.x < 2 * TS * kMqTile) {
+      const int tk = threadIdx.x % (TS * kMqTile), side = (int)threadIdx.x / (TS * kMqTile);
+      buf[(tk / kMqTile) * TILE + kMqTile * (4 * KST + VST) + side * kMqTile + tk % kMqTile] = sc;
+    }
+  };
+
+  constexpr int kStep = kMqTile * TS;
+  load_step(t_begin);
+  if (threadIdx.x < (1 << KB)) s_cbk[threadIdx.x] = cb<KB>(threadIdx.x);
+  if (threadIdx.x < (1 << VB)) s_cbv[threadIdx.x] = cb<VB>(threadIdx.x);
+  // query c16's 8-dim groups 4 i + g (query groups past the last: unused)
+  const bool live = qg < qgroups;
+  float qe[NE];
+  if (live) {
+    const float *qr = qrot + ((size_t)(h * qgroups + qg) * kMqQueries + c16) * P + 8 * g;
+#pragma unroll
+    for (int j = 0; j < NE; ++j) qe[j] = qr[32 * (j / 8) + j % 8];
+  }
+  __syncthreads();
+  store_step(t_begin, s_buf);
+  __syncthreads();
   f32x4 acc[NT];
 #pragma unroll
   for (int i = 0; i < NT; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   float m_run = -INFINITY;  // query c16; the first tile seeds it with the reference's -1e30
   float l_part = 0.0f;      // this lane's tokens' share of query c16's sum
 
-  // K row of this lane's token in the wave's first tile (then prefetched a tile ahead)
-  const int tb0 = t_begin + kMqTile * wave;
-  uint32_t kw[KW];
-  float ksc = 0.0f;
-  if (tb0 < t_end) {
-    const uint32_t slot = (uint32_t)min(tb0 + lane, t_end - 1);
-    load_k_row<P, KB>(d, slot, kw);
-    ksc = d->k_scale[slot];
-  }
-  for (int tb = tb0; tb < t_end; tb += kMqTile * kMqWaves) {
-    // ---- V slices of the lane's 16 tokens (consumed after the logits) ----
-    const bool tvalid = tb + lane < t_end;
-    uint32_t vsl[16];
+  int cur = 0;
+  for (int tb = t_begin; tb < t_end; tb += kStep) {
+    const bool more = tb + kStep < t_end;
+    if (more) load_step(tb + kStep);
+    const float *tile = s_buf + (cur * TS + ts) * TILE;
+    const int tile_tb = tb + ts * kMqTile;
+    if (live && tile_tb < t_end) {
+      // ---- logits (attention.cpp:93-136, :83-88): eight chains ----
+      f32x4 s8[8];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+      for (int L = 0; L < 8; ++L) s8[L] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      const float4 *kr = reinterpret_cast<const float4 *>(tile + (c16 * 4 + g) * KST);
+#pragma unroll
+      for (int j = 0; j < NE / 4; ++j) {
+        const float4 k4 = kr[j];
+        const int L = 4 * (j & 1);
+        s8[L] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.x, qe[4 * j], s8[L], 0, 0, 0);
+        s8[L + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.y, qe[4 * j + 1], s8[L + 1], 0, 0, 0);
+        s8[L + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.z, qe[4 * j + 2], s8[L + 2], 0, 0, 0);
+        s8[L + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.w, qe[4 * j + 3], s8[L + 3], 0, 0, 0);
+      }
+      const float *sc_row = tile + kMqTile * (4 * KST + VST) + 4 * g;
+      const float4 ks4 = *reinterpret_cast<const float4 *>(sc_row);
+      const float4 vs4 = *reinterpret_cast<const float4 *>(sc_row + kMqTile);
+      const float ks[4] = {ks4.x, ks4.y, ks4.z, ks4.w}, vs[4] = {vs4.x, vs4.y, vs4.z, vs4.w};
+      // logits of query c16 and tokens 4 g + r of the tile
+      float lg[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int vs = min(tb + 16 * u + 4 * r + g, t_end - 1);
-        vsl[4 * u + r] = v_slice<P, VB>(vbase + (size_t)vs * v_pb, c16);
+        const float dot = __fadd_rn(
+            __fadd_rn(__fadd_rn(s8[0][r], s8[4][r]), __fadd_rn(s8[1][r], s8[5][r])),
+            __fadd_rn(__fadd_rn(s8[2][r], s8[6][r]), __fadd_rn(s8[3][r], s8[7][r])));
+        lg[r] = __fmul_rn(__fmul_rn(dot, attn_s), ks[r]);
       }
-    // this lane's token's V scale, passed on through the logits' pad column
-    const float vsc_own = tvalid ? d->v_scale[min(tb + lane, t_end - 1)] : 0.0f;
-    float kv[P];
+      if (tile_tb + kMqTile > t_end) {  // tokens past the split's end
 #pragma unroll
-    for (int e = 0; e < P; ++e) kv[e] = s_cbk[code_in<KB>(kw, e)];
-    const float kscale = ksc;
-    // prefetch the next tile's K row
-    const int tn = tb + kMqTile * kMqWaves;
-    if (tn < t_end) {
-      const uint32_t slot = (uint32_t)min(tn + lane, t_end - 1);
-      load_k_row<P, KB>(d, slot, kw);
-      ksc = d->k_scale[slot];
-    }
-
-    // ---- logits (attention.cpp:93-136, :83-88), one query at a time, its
-    // 64-float halves loaded into SGPRs in turn ----
-#pragma unroll 1
-    for (int q = 0; q < kMqQueries; ++q) {
-      const cfloat *qq = qw + q * P;
-      float s8[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int e = 0; e < 64; ++e) s8[e & 7] = fmaf(kv[e], qq[e], s8[e & 7]);
-      if constexpr (P == 128) {
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int e = 64; e < 128; ++e) s8[e & 7] = fmaf(kv[e], qq[e], s8[e & 7]);
+        for (int r = 0; r < 4; ++r) lg[r] = tile_tb + 4 * g + r < t_end ? lg[r] : -INFINITY;
       }
-      const float dot = (__fadd_rn(s8[0], s8[4]) + __fadd_rn(s8[1], s8[5])) +
-                        (__fadd_rn(s8[2], s8[6]) + __fadd_rn(s8[3], s8[7]));
-      s_lg[lane * LST + q] = tvalid ? __fmul_rn(__fmul_rn(dot, attn_s), kscale) : -INFINITY;
-    }
-    s_lg[lane * LST + 16] = vsc_own;
 
-    // ---- to the V product's layout: lane has query c16, tokens 16u + 4r + g ----
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    float lg[4][4], vsc[4][4];
-    float tmax = -1e30f;
+      // ---- online softmax: the maximum moves, and the sums with it, only in
+      // a tile that holds a larger logit (or seeds it) ----
+      const float tmax = fmaxf(fmaxf(lg[0], lg[1]), fmaxf(lg[2], lg[3]));
+      if (__any(tmax > m_run) || tb == t_begin) {
+        const float m_new = fmaxf(m_run, fmaxf(quad_max(tmax), -1e30f));
+        const float alpha = __builtin_amdgcn_exp2f(__fmul_rn(m_run - m_new, kLog2e));
+        m_run = m_new;
+        l_part *= alpha;
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+        for (int r = 0; r < 4; ++r) {
+          // O rows (query 4 g + r of the result layout) by their query's alpha
+          const float a = __shfl(alpha, 4 * g + r, 64);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        lg[u][r] = s_lg[(16 * u + 4 * r + g) * LST + c16];
-        vsc[u][r] = s_lg[(16 * u + 4 * r + g) * LST + 16];
-        tmax = fmaxf(tmax, lg[u][r]);
-      }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();  // the next tile's logits overwrite s_lg
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float m_new = fmaxf(m_run, tmax);
-    const float alpha = __builtin_amdgcn_exp2f(__fmul_rn(m_run - m_new, kLog2e));
-    m_run = m_new;
-    l_part *= alpha;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      // rescale O rows (query 4 g + r of the result layout) by their query's alpha
-      const float a = __shfl(alpha, 4 * g + r, 64);
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[nt][r] *= a;
-    }
-
-    // ---- weighted V: O[q][NT c16 + nt] += sum_t w[q][t] V[t][NT c16 + nt] ----
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float e = __builtin_amdgcn_exp2f(__fmul_rn(lg[u][r] - m_new, kLog2e));
-        l_part += e;
-        const float w = e * vsc[u][r] * isp;
-        const uint32_t sl = vsl[4 * u + r];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          const float v = s_cbv[(sl >> (32 - VB * (nt + 1))) & vmask];
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, v, acc[nt], 0, 0, 0);
+          for (int nt = 0; nt < NT; ++nt) acc[nt][r] *= a;
         }
       }
+
+      // ---- weighted V: O[q][dim] += sum_t w[q][t] V[t][dim], tile nt's column
+      // c16 being dim 64 (nt / 4) + 4 c16 + nt % 4 ----
+      const float *vr = tile + kMqTile * 4 * KST + 4 * g * VST + 4 * c16;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = __builtin_amdgcn_exp2f(__fmul_rn(lg[r] - m_run, kLog2e));
+        l_part += e;
+        const float w = e * vs[r] * isp;
+#pragma unroll
+        for (int b = 0; b < NT / 4; ++b) {
+          const float4 v4 = *reinterpret_cast<const float4 *>(vr + r * VST + 64 * b);
+          acc[4 * b] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, v4.x, acc[4 * b], 0, 0, 0);
+          acc[4 * b + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, v4.y, acc[4 * b + 1], 0, 0, 0);
+          acc[4 * b + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, v4.z, acc[4 * b + 2], 0, 0, 0);
+          acc[4 * b + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, v4.w, acc[4 * b + 3], 0, 0, 0);
+        }
+      }
+    }
+    if constexpr (NBUF == 1) __syncthreads();  // the tiles are read out
+    else cur ^= 1;
+    if (more) store_step(tb + kStep, s_buf + cur * TS * TILE);
+    // the next step's tiles are written; this step's copy is read out.  (At the
+    // loop's end: a barrier at its head, after the store's divergent branches,
+    // was reached by the lanes of a wave one branch at a time.)
+    __syncthreads();
   }
 
-  // ---- merge the waves: record (m, l) of query c16 and acc rows 4 g + r ----
-  __syncthreads();  // every wave is done with its logits
   float l_tot = l_part + __shfl_xor(l_part, 16, 64);
   l_tot += __shfl_xor(l_tot, 32, 64);
+  auto dim_of = [&](int nt) { return 64 * (nt / 4) + 4 * c16 + (nt & 3); };
+  if constexpr (TS == 1) {
+    // the wave's records (m, l) of query c16 and acc rows 4 g + r
+    if (!live) return;
+    if (g == 0 && j0 + c16 < nq) {
+      part_of(j0 + c16)[0] = m_run;
+      part_of(j0 + c16)[1] = l_tot;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (j0 + 4 * g + r < nq) {
+        float *po = part_of(j0 + 4 * g + r) + 4 + 4 * c16;
+#pragma unroll
+        for (int b = 0; b < NT / 4; ++b)
+          *reinterpret_cast<float4 *>(po + 64 * b) = make_float4(
+              acc[4 * b][r], acc[4 * b + 1][r], acc[4 * b + 2][r], acc[4 * b + 3][r]);
+      }
+    return;
+  }
+  // ---- merge the slices of each group (the tiles are read out) ----
   float *rec = s_buf + wave * (kMqQueries * MST);
   if (g == 0) {
     rec[c16 * MST] = m_run;
@@ -386,15 +446,19 @@ __global__ __launch_bounds__(kMqThreads, 1) void decode_mq_kernel(
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) rec[(4 * g + r) * MST + 4 + NT * c16 + nt] = acc[nt][r];
+    for (int nt = 0; nt < NT; ++nt) rec[(4 * g + r) * MST + 4 + dim_of(nt)] = acc[nt][r];
   __syncthreads();
-  for (int i = threadIdx.x; i < kMqQueries * (P + 4); i += kMqThreads) {
-    const int jj = i / (P + 4), e = i - jj * (P + 4);
-    if (j0 + jj >= nq || e == 2 || e == 3) continue;
-    float mw[kMqWaves], M = -INFINITY;
+  for (int i = threadIdx.x; i < QG * kMqQueries * (P + 4); i += kMqThreads) {
+    const int jj = i / (P + 4), e = i - jj * (P + 4), j = qg0 * kMqQueries + jj;
+    if (j >= nq || e == 2 || e == 3) continue;
+    // slice w's record of this query: wave w QG + jj / 16
+    auto rec_of = [&](int w) {
+      return s_buf + ((w * QG + jj / kMqQueries) * kMqQueries + jj % kMqQueries) * MST;
+    };
+    float mw[TS], M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < kMqWaves; ++w) {
-      mw[w] = s_buf[(w * kMqQueries + jj) * MST];
+    for (int w = 0; w < TS; ++w) {
+      mw[w] = rec_of(w)[0];
       M = fmaxf(M, mw[w]);
     }
     float out;
@@ -403,48 +467,68 @@ __global__ __launch_bounds__(kMqThreads, 1) void decode_mq_kernel(
     } else {
       out = 0.0f;
 #pragma unroll
-      for (int w = 0; w < kMqWaves; ++w) {
-        // a wave without tokens has m = -inf and contributes 0
+      for (int w = 0; w < TS; ++w) {
+        // a slice without tokens has m = -inf and contributes 0
         const float f = __builtin_amdgcn_exp2f(__fmul_rn(mw[w] - M, kLog2e));
-        out += s_buf[(w * kMqQueries + jj) * MST + e] * f;
+        out += rec_of(w)[e] * f;
       }
     }
-    part_of(j0 + jj)[e] = out;
+    part_of(j)[e] = out;
   }
 }
 
 struct MqPlan {
   int splits, chunk, qgroups;
+  int qg;       // query groups a block
+  int qblocks;  // blocks over the query groups
 };
 
 MqPlan mq_plan(int n_heads, int nq, int max_n) {
   MqPlan mp;
   mp.qgroups = (nq + kMqQueries - 1) / kMqQueries;
+  mp.qg = mp.qgroups >= 3 ? 4 : mp.qgroups;
+  mp.qblocks = (mp.qgroups + mp.qg - 1) / mp.qg;
   const int max1 = max_n > 0 ? max_n : 1;
-  // about one block per CU (256 blocks), at least one tile per wave
-  constexpr int kStep = kMqTile * kMqWaves;
-  const int blocks = n_heads * mp.qgroups;
-  int splits = (256 + blocks - 1) / blocks;
-  const int by_work = (max1 + kStep - 1) / kStep;
-  splits = std::max(1, std::min(splits, by_work));
+  // two blocks a CU (256 CUs), of at least 128 tokens each.  Measured, 64
+  // queries of 8 heads d128 K4/V4 x 32,768 tokens, the whole call: one block a
+  // CU 147 us, two 129, three (as many as the registers allow) 130 with half
+  // as much finalize work again.
+  const int step = kMqTile * (kMqWaves / mp.qg);
+  const int blocks = n_heads * mp.qblocks;
+  const int splits = std::max(1, std::min(512 / blocks, (max1 + 127) / 128));
   int chunk = (max1 + splits - 1) / splits;
-  chunk = ((chunk + kStep - 1) / kStep) * kStep;
+  chunk = ((chunk + step - 1) / step) * step;
   mp.chunk = chunk;
   mp.splits = (max1 + chunk - 1) / chunk;
   return mp;
 }
 
-// Queries per head from which the matrix-core kernel replaces the LUT
-// kernel's one-query items.
-constexpr int kMqMinQueries = 16;
+// Whether the matrix-core kernel takes nq queries of n_heads heads over max_n
+// tokens, rather than the LUT kernel as nq * n_heads items.  The LUT kernel
+// pays for each query, about 4.5 M values of K a microsecond, in one launch
+// or two; this one for groups of 16 queries, about 11 M values a microsecond,
+// and 10 us more for its rotation and finalize launches.  Measured (whole
+// call, LUT and matrix cores): 8 heads d128 K4/V4 x 32,768 tokens, 4 queries
+// 41 and 51 us, 8 queries 68 and 51, 12 queries 116 and 52; 16 heads d64 K4/V2
+// x 16,384, 8 queries 26 and 31, 12 queries 36 and 32; 2 heads d128 K3/V3 x
+// 32,768, 12 queries 39 and 38; 12 heads d128 x 512, 12 queries 9 and 18; 4
+// heads d64 x 1,024, 12 queries 7 and 14.
+constexpr int kMqMinQueries = 8;
+
+bool mq_pays(int n_heads, int nq, const DecodeShape &sh) {
+  if (nq < kMqMinQueries) return false;
+  const double per_query = (double)n_heads * (sh.max_n > 0 ? sh.max_n : 1) * sh.padded;
+  const int padded_nq = (nq + kMqQueries - 1) / kMqQueries * kMqQueries;
+  return nq * per_query / 4.5e6 > 10.0 + padded_nq * per_query / 1.1e7;
+}
 
 bool mq_eligible(int n_items, int n_heads, const DecodeShape &sh) {
   if (n_heads <= 0 || n_items % n_heads != 0) return false;
   const int nq = n_items / n_heads;
   const bool kq = sh.k_bits >= 2 && sh.k_bits <= 4, vq = sh.v_bits >= 2 && sh.v_bits <= 4;
-  return !sh.raw && kq && vq && (sh.padded == 64 || sh.padded == 128) && nq >= kMqMinQueries &&
-         n_heads <= 65535 && (int64_t)n_heads * ((nq + kMqQueries - 1) / kMqQueries) *
-                                      ((sh.max_n + kMqTile * kMqWaves - 1) / (kMqTile * kMqWaves)) <
+  return !sh.raw && kq && vq && (sh.padded == 64 || sh.padded == 128) &&
+         mq_pays(n_heads, nq, sh) && n_heads <= 65535 && (int64_t)n_heads * ((nq + kMqQueries - 1) / kMqQueries) *
+                                      ((sh.max_n + 127) / 128) <
                                   (int64_t)1 << 31;
 }
 
@@ -455,16 +539,21 @@ hipError_t dispatch_mq(const DecodeShape &sh, dim3 grid, HeadDesc *const *descs,
   mq_rotate_kernel<P><<<dim3((mp.qgroups * kMqQueries + 3) / 4, n_heads), 256, 0, s>>>(
       descs, n_heads, nq, mp.qgroups, q, qrot);
   if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+#define AQ_MQ_QG(KB_, VB_, QG_)                                                             \
+  decode_mq_kernel<P, KB_, VB_, QG_><<<grid, kMqThreads, 0, s>>>(                           \
+      descs, n_heads, nq, mp.qgroups, mp.chunk, mp.splits, qrot, part)
 #define AQ_MQ(KB_, VB_)                                                                     \
   if (sh.k_bits == KB_ && sh.v_bits == VB_) {                                               \
-    decode_mq_kernel<P, KB_, VB_><<<grid, kMqThreads, 0, s>>>(descs, n_heads, nq, mp.qgroups, \
-                                                              mp.chunk, mp.splits, qrot, part); \
+    if (mp.qg == 4) AQ_MQ_QG(KB_, VB_, 4);                                                  \
+    else if (mp.qg == 2) AQ_MQ_QG(KB_, VB_, 2);                                             \
+    else AQ_MQ_QG(KB_, VB_, 1);                                                             \
     return hipGetLastError();                                                               \
   }
   AQ_MQ(4, 2) AQ_MQ(4, 3) AQ_MQ(4, 4)
   AQ_MQ(3, 2) AQ_MQ(3, 3) AQ_MQ(3, 4)
   AQ_MQ(2, 2) AQ_MQ(2, 3) AQ_MQ(2, 4)
 #undef AQ_MQ
+#undef AQ_MQ_QG
   return hipErrorInvalidValue;
 }
 
@@ -490,7 +579,7 @@ hipError_t launch_decode_multi(HeadDesc *const *descs, int n_items, int n_heads,
     return launch_decode(descs, n_items, sh, d_q, d_out, d_ws, s);
   const int nq = n_items / n_heads;
   const MqPlan mp = mq_plan(n_heads, nq, sh.max_n);
-  const dim3 grid(mp.splits * n_heads * mp.qgroups);
+  const dim3 grid((unsigned)mp.splits * n_heads * mp.qblocks);
   float *qrot = d_ws, *part = d_ws + mq_qrot_floats(n_heads, mp, sh.padded);
   const hipError_t e =
       sh.padded == 64 ? dispatch_mq<64>(sh, grid, descs, n_heads, nq, mp, d_q, qrot, part, s)
