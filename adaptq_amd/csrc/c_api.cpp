@@ -1550,15 +1550,30 @@ int adaptq_ggml_attn_f32_device(adaptq_mha_t h, const float *d_q, int head_dim, 
   const int H = m->n_heads;
   DeviceGuard g(m->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const size_t rows = (size_t)n_queries * H;
-  const size_t io = align256(rows * head_dim * 4);
-  if (hip_fail(m->d_io.ensure(2 * io), fn)) return -1;
-  float *dq = static_cast<float *>(m->d_io.p);
-  float *dout = reinterpret_cast<float *>(static_cast<uint8_t *>(m->d_io.p) + io);
-  // queries as [query][head][dim]
-  if (hip_fail(caller_begin(m->device, s), fn) ||
-      hip_fail(aq::launch_gather_rows(dq, d_q, n_queries, H, head_dim, q_nb2, q_nb1, s), fn))
-    return -1;
+  const size_t rows = (size_t)n_queries * H, bytes = rows * head_dim * 4;
+  // Rows that already lie [query][head][dim] on both sides are read and
+  // written in place; a destination that overlaps the queries other than
+  // exactly (each decode reads its query before it writes its output) and any
+  // other stride go through copies (a launch of about 5 us each way).
+  auto packed = [&](size_t nb1, size_t nb2) {
+    return (H == 1 || nb1 == (size_t)head_dim * 4) &&
+           (n_queries == 1 || nb2 == (size_t)H * head_dim * 4);
+  };
+  const uintptr_t qa = reinterpret_cast<uintptr_t>(d_q), da = reinterpret_cast<uintptr_t>(d_dst);
+  const bool direct = packed(q_nb1, q_nb2) && packed(d_nb1, d_nb2) &&
+                      (qa == da || qa + bytes <= da || da + bytes <= qa);
+  const float *dq = d_q;
+  float *dout = d_dst;
+  if (hip_fail(caller_begin(m->device, s), fn)) return -1;
+  if (!direct) {
+    const size_t io = align256(bytes);
+    if (hip_fail(m->d_io.ensure(2 * io), fn)) return -1;
+    float *rows_in = static_cast<float *>(m->d_io.p);
+    dout = reinterpret_cast<float *>(static_cast<uint8_t *>(m->d_io.p) + io);
+    if (hip_fail(aq::launch_gather_rows(rows_in, d_q, n_queries, H, head_dim, q_nb2, q_nb1, s), fn))
+      return -1;
+    dq = rows_in;
+  }
   const int n = launch_all_locked(m, dq, dout, s, fn, n_queries);
   if (n == -2) {
     set_error("adaptq_ggml_attn_f32_device: heads differ in ring size or branch; "
@@ -1566,9 +1581,10 @@ int adaptq_ggml_attn_f32_device(adaptq_mha_t h, const float *d_q, int head_dim, 
     return -1;
   }
   if (n < 0) return -1;
-  if (hip_fail(aq::launch_scatter_rows(d_dst, dout, n_queries, H, head_dim, d_nb2, d_nb1, s), fn) ||
-      hip_fail(caller_end(m->device, s), fn))
+  if (!direct &&
+      hip_fail(aq::launch_scatter_rows(d_dst, dout, n_queries, H, head_dim, d_nb2, d_nb1, s), fn))
     return -1;
+  if (hip_fail(caller_end(m->device, s), fn)) return -1;
   return n;
 }
 
