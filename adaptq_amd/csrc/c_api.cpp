@@ -748,6 +748,7 @@ struct Plan {
   std::mutex mu;          // one call on the plan at a time
   uint64_t seen = 0;      // epoch the cache below was read at (0: never)
   int max_n = 0;          // largest ring size
+  long long sum_n = 0;    // sum of the ring sizes
   Mode mode = Mode::Dense;
   bool mixed = false;     // non-empty contexts take different branches
 };
@@ -760,6 +761,7 @@ bool plan_scan(Plan *p, const char *fn, bool flush = true) {
   if (p->seen != 0 && g_epoch.load(std::memory_order_acquire) == p->seen) return true;
   const uint64_t e0 = g_epoch.load(std::memory_order_acquire);
   int max_n = 0;
+  long long sum_n = 0;
   bool have = false, mixed = false;
   Mode mode = Mode::Dense;
   for (Ctx *c : p->ctxs) {
@@ -776,44 +778,53 @@ bool plan_scan(Plan *p, const char *fn, bool flush = true) {
       have = true;
     }
     max_n = std::max(max_n, c->st.size);
+    sum_n += c->st.size;
   }
   p->max_n = max_n;
+  p->sum_n = sum_n;
   p->mode = mode;
   p->mixed = mixed;
   p->seen = e0;
   return true;
 }
 
+// The plan's decode: rings of uneven length are split by the sum of their
+// sizes.
+aq::DecodeShape plan_shape(const Plan *p, bool one_split) {
+  const Ctx *c0 = p->ctxs[0];
+  aq::DecodeShape sh{c0->dim, c0->padded, c0->k_bits, c0->v_bits, p->mode == Mode::Hybrid,
+                     p->max_n};
+  if (p->sum_n < (long long)p->max_n * (long long)p->ctxs.size()) sh.sum_n = p->sum_n;
+  sh.one_split = one_split;
+  return sh;
+}
+
 // The batched decode of a plan on stream s (caller holds p->mu and has
-// scanned).  d_ws: workspace of at least ws_floats floats.
+// scanned).  d_ws: workspace of at least plan_ws_floats(p, one_split) floats.
 int plan_launch_decode(Plan *p, const float *d_queries, float *d_outs, float *d_ws,
-                       hipStream_t s, const char *fn) {
+                       hipStream_t s, const char *fn, bool one_split = false) {
   if (p->mixed) {
     set_error(
         "adaptq_plan_compute_device: contexts take different branches (dense, sparse-V, "
         "hybrid); use one plan per branch or adaptq_compute");
     return -1;
   }
-  const Ctx *c0 = p->ctxs[0];
   const int n_items = (int)p->ctxs.size();
-  aq::DecodeShape sh{c0->dim, c0->padded, c0->k_bits, c0->v_bits, p->mode == Mode::Hybrid,
-                     p->max_n};
+  const aq::DecodeShape sh = plan_shape(p, one_split);
   auto **items = static_cast<aq::HeadDesc **>(p->d_list.p);
   hipError_t e = caller_begin(p->device, s);
   if (e == hipSuccess)
     e = p->mode == Mode::Sparse && p->max_n > 0
-            ? aq::launch_decode_sparse(items, n_items, sh, c0->v_mass, d_queries, d_outs, d_ws, s)
+            ? aq::launch_decode_sparse(items, n_items, sh, p->ctxs[0]->v_mass, d_queries, d_outs, d_ws, s)
             : aq::launch_decode(items, n_items, sh, d_queries, d_outs, d_ws, s);
   if (e == hipSuccess) e = caller_end(p->device, s);
   if (hip_fail(e, fn)) return -1;
   return 0;
 }
 
-size_t plan_ws_floats(const Plan *p) {
-  const Ctx *c0 = p->ctxs[0];
+size_t plan_ws_floats(const Plan *p, bool one_split = false) {
   const int n_items = (int)p->ctxs.size();
-  aq::DecodeShape sh{c0->dim, c0->padded, c0->k_bits, c0->v_bits, p->mode == Mode::Hybrid,
-                     p->max_n};
+  const aq::DecodeShape sh = plan_shape(p, one_split);
   return p->mode == Mode::Sparse && p->max_n > 0 ? aq::sparse_workspace_floats(n_items, sh)
                                                  : aq::decode_workspace_floats(n_items, sh);
 }
@@ -901,9 +912,12 @@ int launch_all_locked(Mha *m, const float *dq, float *dout, hipStream_t s, const
   const int H = m->n_heads * reps;
   aq::DecodeShape sh{c0->dim, c0->padded, c0->k_bits, c0->v_bits, mode == Mode::Hybrid,
                      n > 0 ? n : 1};
-  const size_t wsf = mode == Mode::Sparse ? aq::sparse_workspace_floats(H, sh)
-                                          : aq::decode_multi_workspace_floats(H, m->n_heads, sh);
-  if (hip_fail(m->d_ws.ensure(wsf * 4), fn)) return -1;
+  auto ws_bytes = [&] {
+    return 4 * (mode == Mode::Sparse ? aq::sparse_workspace_floats(H, sh)
+                                     : aq::decode_multi_workspace_floats(H, m->n_heads, sh));
+  };
+  sh.one_split = ws_bytes() > m->d_ws.bytes && capturing(s);  // as a plan's decode
+  if (hip_fail(m->d_ws.ensure(ws_bytes()), fn)) return -1;
   auto **items = static_cast<aq::HeadDesc **>(m->d_list.p);
   if (reps > 1) {
     if (m->rep_n != reps) {
@@ -1773,6 +1787,7 @@ int adaptq_plan_append_device(adaptq_plan_t h, const float *d_keys, const float 
   // the plan's cache in one pass, without the contexts' locks (calls that
   // touch the same contexts must not overlap a plan call).
   int max_n = 0;
+  long long sum_n = 0;
   bool have = false, mixed = false;
   Mode mode = Mode::Dense;
   for (Ctx *c : p->ctxs) {
@@ -1784,8 +1799,10 @@ int adaptq_plan_append_device(adaptq_plan_t h, const float *d_keys, const float 
       have = true;
     }
     max_n = std::max(max_n, c->st.size);
+    sum_n += c->st.size;
   }
   p->max_n = max_n;
+  p->sum_n = sum_n;
   p->mode = mode;
   p->mixed = mixed;
   // the states changed: other plans over these contexts must rescan; this
@@ -1861,9 +1878,12 @@ int adaptq_plan_compute_device(adaptq_plan_t h, const float *d_queries, float *d
   std::lock_guard<std::mutex> gp(p->mu);
   if (!plan_scan(p, fn)) return -1;
   DeviceGuard g(p->device);
-  if (!p->mixed && hip_fail(p->d_ws.ensure(plan_ws_floats(p) * 4), fn)) return -1;
-  return plan_launch_decode(p, d_queries, d_outs, static_cast<float *>(p->d_ws.p),
-                            static_cast<hipStream_t>(stream), fn);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  // nothing may be allocated under graph capture: a decode whose splits have
+  // no workspace yet runs unsplit there where it can
+  const bool one_split = !p->mixed && plan_ws_floats(p) * 4 > p->d_ws.bytes && capturing(s);
+  if (!p->mixed && hip_fail(p->d_ws.ensure(plan_ws_floats(p, one_split) * 4), fn)) return -1;
+  return plan_launch_decode(p, d_queries, d_outs, static_cast<float *>(p->d_ws.p), s, fn, one_split);
 }
 
 }  // extern "C"

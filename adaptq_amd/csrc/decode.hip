@@ -737,7 +737,8 @@ __global__ __launch_bounds__(kLutThreads, P <= 128 && (KB == 2 || KB == 4) ? 4 :
   float *s_vlut = reinterpret_cast<float *>(s_mem);
   float *s_klut = reinterpret_cast<float *>(s_mem + kVlutBytes);
 
-  const int item = blockIdx.y, split = blockIdx.x;
+  // items fastest (see launch_decode_items)
+  const int item = blockIdx.x, split = blockIdx.y;
   // Descriptor fields are read through the constant address space so they
   // load as scalars (a generic-pointer load is assumed divergent).
   const AQ_AS4 HeadDesc *d =
@@ -1839,6 +1840,48 @@ SplitPlan plan_splits(int n_items, int max_n, int min_chunk, int target_blocks) 
   return sp;
 }
 
+// Splits of the LUT kernel, by estimated time in tokens of one 512-thread
+// block alone on a CU.  A block's fixed work (query rotation, K table, merge)
+// is worth kBlock tokens (1,500 at padded 128; half with 3-bit keys, whose
+// table is a quarter of the others') and the finalize launch kFinal; two blocks on a CU run 1.16 times as fast together, each 1.72 times as
+// long while both last (1.3 assumed of the longest).  Up to 256 blocks the
+// longest decides, above it that or the sum over the CUs and an uneven end.  The estimate only ranks split counts;
+// measured (us, chosen split first): 48 items x 32,768 tokens d128 K4/V4 in 5
+// splits 58, in 6 68; 100 x 4,096 d128 K4/V2 in 2 splits 18.8, in 3 20.0; 8 x
+// 32,768 in 32 splits 19.8, in 16 24.8, in 64 21.7; 336 x 4,096 in 1 split
+// 35.0, in 2 35.3; 512 items of 256 to 6,746 tokens (log-uniform) d96 K3/V3 in
+// 3 splits 50, in 1 65.6, d128 K4/V2 in 2 splits 38, in 1 42.5.
+SplitPlan plan_lut(int n_items, int max_n, const DecodeShape &sh) {
+  const double kBlock = (sh.k_bits == 3 ? 750.0 : 1500.0) * 128 / sh.padded;
+  const double kFinal = 800.0 * 128 / sh.padded;
+  const bool even = sh.sum_n <= 0;
+  const double sum = even ? (double)n_items * max_n : (double)sh.sum_n;
+  const int most = (max_n + kLutWaves * kTile - 1) / (kLutWaves * kTile);
+  SplitPlan best{1, (max_n + kTile - 1) / kTile * kTile};
+  double best_t = 0.0;
+  for (int s = 1; s <= most; s += s < 8 ? 1 : s / 8) {
+    // (the workspace stays within the 8 MiB that the allocation-free call
+    // has: unsplit, a plan needs none)
+    if (s > 1 && (sh.one_split || (double)n_items * s * (sh.padded + 4) * 4 > (double)(8 << 20)))
+      break;
+    // whole rounds of the block's waves: a chunk of 4.5 takes 5
+    const int unit = s > 1 ? kLutWaves * kTile : kTile;
+    const int chunk = ((max_n + s - 1) / s + unit - 1) / unit * unit;
+    const int splits = (max_n + chunk - 1) / chunk;
+    const double blocks = even ? (double)n_items * splits
+                               : sum / chunk + (splits > 1 ? 0.5 * n_items : 0.0);
+    const double n_blocks = blocks > n_items ? blocks : n_items;
+    const double one = chunk + kBlock, all = (sum + n_blocks * kBlock) / (256 * 1.163);
+    double t = n_blocks <= 256 ? one : std::max(1.3 * one, all + 0.5 * one);
+    if (splits > 1) t += kFinal + 10.0 * splits;
+    if (s == 1 || t < best_t) {
+      best_t = t;
+      best = SplitPlan{splits, chunk};
+    }
+  }
+  return best;
+}
+
 template <int P, bool RAW>
 hipError_t dispatch_lut(const DecodeShape &sh, dim3 grid, HeadDesc *const *descs, const float *q,
                         int chunk, int splits, float *part, float *out, hipStream_t s) {
@@ -1956,12 +1999,7 @@ SplitPlan decode_plan(int n_items, const DecodeShape &sh) {
     sp.chunk = ((max_n + kTile - 1) / kTile) * kTile;
     return sp;
   }
-  // LUT kernel: about one 512-thread block per CU (256 CUs): each extra block
-  // repeats the query rotation and the K table build, and the splits add
-  // finalize work (measured: 4 heads x 131,072 tokens 48 -> 27 us, 64 heads x
-  // 8,192 tokens 35 -> 25 us, 8 heads x 32,768 tokens 28 -> 25 us against a
-  // target of 1,024 blocks; none of the sampled shapes slower).
-  if (lut) return plan_splits(n_items, max_n, kLutWaves * kTile, 256);
+  if (lut) return plan_lut(n_items, max_n, sh);
   // wide kernel: each block builds a table of 2^KB x P entries, so a block
   // takes at least 512 tokens; 4 blocks a CU at padded 512 (a 4-bit table
   // takes 36 KB of LDS), 2 at padded 1024 (68 KB)
@@ -2056,7 +2094,7 @@ hipError_t launch_decode_step(HeadDesc *const *descs, int n_items, const DecodeS
   if (n_items <= 0) return hipSuccess;
   if (!decode_step_supported(n_items, sh)) return hipErrorNotSupported;
   const SplitPlan sp = decode_plan(n_items, sh);
-  const dim3 grid(1, n_items);
+  const dim3 grid(n_items, 1);
   return dispatch_lut_step<64>(sh, grid, descs, d_q, sp.chunk, d_out, app, s);
 }
 
@@ -2068,6 +2106,11 @@ hipError_t launch_decode_items(HeadDesc *const *descs, int n_items, const Decode
   const dim3 grid(sp.splits, n_items);
   hipError_t e;
   if (lut_ok) {
+    // items fastest: consecutive blocks go to the 8 XCDs in turn, and with
+    // splits fastest a split count that shares a factor with 8 puts the last
+    // splits of every item (empty ones, where rings differ in length) on the
+    // same XCDs and the first ones on the others
+    const dim3 grid(n_items, sp.splits);
     if (sh.padded == 64)
       e = raw ? dispatch_lut<64, true>(sh, grid, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s)
               : dispatch_lut<64, false>(sh, grid, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s);

@@ -32,6 +32,10 @@ struct DecodeShape {
   int dim, padded, k_bits, v_bits;
   bool raw;   // hybrid branch: exact fp32 attention over the raw mirror
   int max_n;  // largest ring size among the items (host view)
+  long long sum_n = 0;  // sum of the items' ring sizes; 0: all are max_n
+  // whether the LUT kernel takes one block per item, which needs no workspace
+  // (a call that may not allocate any)
+  bool one_split = false;
 };
 
 // Floats of workspace the decode of n_items items needs.

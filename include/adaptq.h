@@ -306,8 +306,8 @@ int adaptq_plan_compute_device_static(adaptq_plan_t plan, const float *d_queries
  * when its contexts take different branches): what
  * adaptq_plan_compute_device allocates and adaptq_plan_compute_device_static
  * takes from its 8 MiB array.  Dense plans need none when each context's ring
- * fits one block per item (about 512 contexts or more at padded 64/128), else
- * (padded + 4) * 4 bytes per context and split; sparse-V plans need about
+ * fits one block per item (about 512 contexts or more of even length at padded
+ * 64/128), else (padded + 4) * 4 bytes per context and split, up to 8 MiB; sparse-V plans need about
  * 4 + 4 * padded / 256 bytes per token of the longest ring per context up to
  * 8,192 tokens, and about 22 + 4 * padded / 256 bytes per token above.
  * Returns -1 on error (a null handle, or a context with staged host
