@@ -91,6 +91,17 @@ class PyMHAContext {
     return n;
   }
 
+  // Append one token and decode one query for every head (rows of io_type).
+  int step_device(uintptr_t d_keys, uintptr_t d_vals, uintptr_t d_queries, uintptr_t d_outs,
+                  int io_type, int pos, uintptr_t stream) {
+    const int n = adaptq_mha_step_device(
+        backend_.handle(), reinterpret_cast<const void *>(d_keys),
+        reinterpret_cast<const void *>(d_vals), reinterpret_cast<const void *>(d_queries),
+        reinterpret_cast<void *>(d_outs), io_type, pos, reinterpret_cast<void *>(stream));
+    if (n < 0) throw std::runtime_error(adaptq_last_error());
+    return n;
+  }
+
   void reset() { backend_.reset(); }
   size_t kv_bytes() const { return backend_.kv_bytes(); }
   int n_heads() const { return n_heads_; }
@@ -120,6 +131,9 @@ PYBIND11_MODULE(adaptq_py, m) {
            py::arg("d_vals"), py::arg("n_tokens"), py::arg("pos"), py::arg("stream"))
       .def("compute_all_device", &PyMHAContext::compute_all_device, py::arg("d_queries"),
            py::arg("d_outs"), py::arg("stream"))
+      .def("step_device", &PyMHAContext::step_device, py::arg("d_keys"), py::arg("d_vals"),
+           py::arg("d_queries"), py::arg("d_outs"), py::arg("io_type"), py::arg("pos"),
+           py::arg("stream"))
       .def("reset", &PyMHAContext::reset)
       .def("kv_bytes", &PyMHAContext::kv_bytes)
       .def_property_readonly("n_heads", &PyMHAContext::n_heads)

@@ -972,6 +972,86 @@ int step_all_locked(Mha *m, const float *dk, const float *dv, const float *dq, f
   return a0.size;
 }
 
+// The same on the hybrid branch, in one launch (launch_mirror_step), for rows
+// of any IoType: when every head's mirror holds the same tokens, all of its
+// ring, after the append.  Returns -2, having launched nothing, when it does
+// not; the common ring size, or -1.
+int mirror_step_locked(Mha *m, const void *dk, const void *dv, const void *dq, void *dout,
+                       aq::IoType io, hipStream_t s, const char *fn) {
+  const Ctx *c0 = m->heads[0];
+  const aq::RingState a0 = aq::ring_after(c0->st, 1, c0->cap, c0->hyb);
+  if (!aq::mirror_step_supported(m->n_heads, c0->padded, a0.size)) return -2;
+  for (const Ctx *c : m->heads) {
+    const aq::RingState a = aq::ring_after(c->st, 1, c->cap, c->hyb);
+    if (c->staged != 0 || a.size != a0.size || mode_at(c, a) != Mode::Hybrid) return -2;
+  }
+  if (hip_fail(aq::launch_mirror_step(static_cast<aq::HeadDesc **>(m->d_list.p), m->n_heads,
+                                      c0->padded, c0->k_bits, c0->v_bits, c0->dim, dk, dv, dq,
+                                      dout, io, s),
+               fn))
+    return -1;
+  for (Ctx *c : m->heads) c->st = aq::ring_after(c->st, 1, c->cap, c->hyb);
+  bump_epoch();
+  return a0.size;
+}
+
+// One token appended to every head and one query each, on a caller's stream:
+// one launch where a fused step takes it, else an append launch and the
+// decode's; rows that are not fp32 are converted around those in scratch
+// memory of the MHA.
+int step_device(Mha *m, const void *dk, const void *dv, const void *dq, void *dout, aq::IoType io,
+                hipStream_t s, const char *fn) {
+  std::lock_guard<std::mutex> gm(m->mu);
+  HeadLocks locks(m);
+  if (!flush_all_locked(m, fn)) return -1;
+  DeviceGuard g(m->device);
+  if (hip_fail(caller_begin(m->device, s), fn)) return -1;
+  int n = mirror_step_locked(m, dk, dv, dq, dout, io, s, fn);
+  if (n == -2) {
+    const Ctx *c0 = m->heads[0];
+    const size_t count = (size_t)m->n_heads * c0->dim;
+    const float *k = static_cast<const float *>(dk), *v = static_cast<const float *>(dv);
+    const float *q = static_cast<const float *>(dq);
+    float *o = static_cast<float *>(dout);
+    if (io != aq::IoType::F32) {
+      const size_t each = align256(count * 4);
+      if (hip_fail(m->d_io.ensure(4 * each), fn)) return -1;
+      auto at = [&](int i) {
+        return reinterpret_cast<float *>(static_cast<uint8_t *>(m->d_io.p) + i * each);
+      };
+      float *const dst[3] = {at(0), at(1), at(2)};
+      const void *const src[3] = {dk, dv, dq};
+      if (hip_fail(aq::launch_to_f32(dst, src, 3, count, io, s), fn)) return -1;
+      k = dst[0];
+      v = dst[1];
+      q = dst[2];
+      o = at(3);
+    }
+    n = step_all_locked(m, k, v, q, o, s, fn);
+    if (n == -2) {  // the append and the decode as two launches
+      if (hip_fail(aq::launch_append(static_cast<aq::HeadDesc **>(m->d_list.p), m->n_heads,
+                                     c0->dim, c0->padded, c0->k_bits, c0->v_bits, k, v, 1, s,
+                                     any_mirror(m->heads, 1)),
+                   fn))
+        return -1;
+      for (Ctx *c : m->heads) c->st = aq::ring_after(c->st, 1, c->cap, c->hyb);
+      bump_epoch();
+      n = launch_all_locked(m, q, o, s, fn);
+      if (n == -2) {
+        (void)caller_end(m->device, s);
+        set_errorf(fn, "heads differ in ring size or branch (the token was appended); use "
+                       "adaptq_mha_compute_all");
+        return -1;
+      }
+    }
+    if (n >= 0 && io != aq::IoType::F32 &&
+        hip_fail(aq::launch_from_f32(dout, o, count, io, s), fn))
+      return -1;
+  }
+  if (n >= 0 && hip_fail(caller_end(m->device, s), fn)) return -1;
+  return n;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1360,33 +1440,25 @@ int adaptq_mha_append_compute_all_device(adaptq_mha_t h, const float *d_keys,
       !require_pointer(d_vals, fn, "d_vals") || !require_pointer(d_queries, fn, "d_queries") ||
       !require_pointer(d_outs, fn, "d_outs"))
     return -1;
-  Mha *m = static_cast<Mha *>(h);
-  std::lock_guard<std::mutex> gm(m->mu);
-  HeadLocks locks(m);
-  if (!flush_all_locked(m, fn)) return -1;
-  DeviceGuard g(m->device);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (hip_fail(caller_begin(m->device, s), fn)) return -1;
-  int n = step_all_locked(m, d_keys, d_vals, d_queries, d_outs, s, fn);
-  if (n == -2) {  // the append and the decode as two launches
-    const Ctx *c0 = m->heads[0];
-    if (hip_fail(aq::launch_append(static_cast<aq::HeadDesc **>(m->d_list.p), m->n_heads, c0->dim,
-                                   c0->padded, c0->k_bits, c0->v_bits, d_keys, d_vals, 1, s,
-                                   any_mirror(m->heads, 1)),
-                 fn))
-      return -1;
-    for (Ctx *c : m->heads) c->st = aq::ring_after(c->st, 1, c->cap, c->hyb);
-    bump_epoch();
-    n = launch_all_locked(m, d_queries, d_outs, s, fn);
-    if (n == -2) {
-      (void)caller_end(m->device, s);
-      set_error("adaptq_mha_append_compute_all_device: heads differ in ring size or branch "
-                "(the token was appended); use adaptq_mha_compute_all");
-      return -1;
-    }
+  return step_device(static_cast<Mha *>(h), d_keys, d_vals, d_queries, d_outs, aq::IoType::F32,
+                     static_cast<hipStream_t>(stream), fn);
+}
+
+int adaptq_mha_step_device(adaptq_mha_t h, const void *d_keys, const void *d_vals,
+                           const void *d_queries, void *d_outs, int io_type, int token_pos,
+                           void *stream) {
+  (void)token_pos;
+  const char *fn = "adaptq_mha_step_device";
+  if (!require_handle(h, fn) || !require_pointer(d_keys, fn, "d_keys") ||
+      !require_pointer(d_vals, fn, "d_vals") || !require_pointer(d_queries, fn, "d_queries") ||
+      !require_pointer(d_outs, fn, "d_outs"))
+    return -1;
+  if (io_type < ADAPTQ_IO_F32 || io_type > ADAPTQ_IO_BF16) {
+    set_error("adaptq_mha_step_device: io_type must be ADAPTQ_IO_F32, _F16 or _BF16");
+    return -1;
   }
-  if (n >= 0 && hip_fail(caller_end(m->device, s), fn)) return -1;
-  return n;
+  return step_device(static_cast<Mha *>(h), d_keys, d_vals, d_queries, d_outs,
+                     static_cast<aq::IoType>(io_type), static_cast<hipStream_t>(stream), fn);
 }
 
 // ---- ggml operator forms (GGML_OP_ADAPTQ_APPEND / GGML_OP_ADAPTQ_ATTN) ----

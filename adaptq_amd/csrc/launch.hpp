@@ -61,6 +61,24 @@ hipError_t launch_decode_step(HeadDesc *const *d_item_desc, int n_items, const D
 // Whether launch_decode_step takes n_items items of this shape.
 bool decode_step_supported(int n_items, const DecodeShape &shape);
 
+// Number type of the rows a step takes and gives.
+enum class IoType { F32 = 0, F16 = 1, BF16 = 2 };
+
+// A decode step on the hybrid branch in one launch: append token k/v [item][dim]
+// to item i's ring and fp32 mirror (as launch_append with one token), then
+// attend over the mirror, the new token included.  n: tokens after the append,
+// the same for every item and all in the mirror.  Rows, queries and outputs of
+// type io.
+bool mirror_step_supported(int n_items, int padded, int n);
+hipError_t launch_mirror_step(HeadDesc *const *d_item_desc, int n_items, int padded, int k_bits,
+                              int v_bits, int dim, const void *k, const void *v, const void *q,
+                              void *out, IoType io, hipStream_t stream);
+
+// n values of type io -> fp32 for up to three arrays in one launch, and back.
+hipError_t launch_to_f32(float *const dst[3], const void *const src[3], int n_arrays, size_t n,
+                         IoType io, hipStream_t stream);
+hipError_t launch_from_f32(void *dst, const float *src, size_t n, IoType io, hipStream_t stream);
+
 // Merge of split partials (m, l, acc[padded]) per item, laid out
 // [item][split][padded + 4], into outputs [item][dim]: log-sum-exp weights,
 // normalisation, inverse FWHT and signs when V is quantised.

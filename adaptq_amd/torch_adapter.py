@@ -4,9 +4,9 @@ over the GPU KV cache.
 Same constructor, ``forward(q, k, v)`` on (1, heads, dim) tensors and
 ``reset_cache()``.  The reference moves every tensor to the CPU and back
 (torch_adapter.py:100-108); here tensors on a ROCm device stay there: the
-step appends k, v and decodes q through the whole-MHA device entry points on
-torch's current stream, so no host copy is made.  CPU tensors take the
-Engine's host path.
+step appends k, v and decodes q in one call on torch's current stream, in
+their own element type (fp32, fp16 or bf16), so nothing is copied to the host.
+CPU tensors take the Engine's host path.
 """
 from __future__ import annotations
 
@@ -14,6 +14,10 @@ import torch
 import torch.nn as nn
 
 from .core import Engine
+
+
+# element types that the step reads and writes itself (ADAPTQ_IO_* in adaptq.h)
+_IO_TYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
 
 class AdaptQAttention(nn.Module):
@@ -47,16 +51,18 @@ class AdaptQAttention(nn.Module):
             raise ValueError(f"Expected v shape {tuple(q.shape)}, got {tuple(v.shape)}.")
 
         if q.is_cuda:
-            kd = k.detach()[0].to(torch.float32).contiguous()
-            vd = v.detach()[0].to(torch.float32).contiguous()
-            qd = q.detach()[0].to(torch.float32).contiguous()
-            out = torch.empty_like(qd)
-            stream = torch.cuda.current_stream(q.device).cuda_stream
-            ctx = self.engine._ctx
-            ctx.append_all_device(kd.data_ptr(), vd.data_ptr(), 1, self.engine.pos, stream)
+            io = _IO_TYPES.get(q.dtype, 0)
+            if k.dtype == q.dtype == v.dtype and q.dtype in _IO_TYPES:
+                qd, kd, vd = (x.detach().contiguous() for x in (q, k, v))
+            else:
+                qd, kd, vd = (x.detach().to(torch.float32).contiguous() for x in (q, k, v))
+                io = 0
+            out = torch.empty(q.shape, dtype=qd.dtype, device=q.device)
+            self.engine._ctx.step_device(kd.data_ptr(), vd.data_ptr(), qd.data_ptr(),
+                                         out.data_ptr(), io, self.engine.pos,
+                                         torch.cuda.current_stream(q.device).cuda_stream)
             self.engine.pos += 1
-            ctx.compute_all_device(qd.data_ptr(), out.data_ptr(), stream)
-            return out.unsqueeze(0).to(dtype=q.dtype)
+            return out if out.dtype == q.dtype else out.to(dtype=q.dtype)
 
         k_np = k.detach().float().cpu().numpy()[0]
         v_np = v.detach().float().cpu().numpy()[0]

@@ -190,7 +190,8 @@ int adaptq_mha_compute_all_device(adaptq_mha_t mha, const float *d_queries,
  * adaptq_mha_compute_all_device (d_queries -> d_outs, device [n_heads][dim]),
  * asynchronous on `stream`.  Same ring bytes and outputs as those two calls
  * (attention.cpp:338-366 then :480-660); where the step is a dense decode at
- * padded 64 with quantised K and V and one block per head, the append runs
+ * padded 64 with quantised K and V and one block per head, or a decode over
+ * the hybrid mirror (up to 512 tokens, padded 64 to 256), the append runs
  * inside the decode launch (one launch instead of two).  Returns the ring
  * size after the append, or -1 (the token is appended when only the decode
  * fails, e.g. heads that differ in ring size or branch). */
@@ -198,6 +199,20 @@ int adaptq_mha_append_compute_all_device(adaptq_mha_t mha, const float *d_keys,
                                          const float *d_vals, int token_pos,
                                          const float *d_queries, float *d_outs,
                                          void *stream);
+
+/* Extension, no counterpart in the reference.  The same step for rows that a
+ * framework holds in half precision (d_keys, d_vals, d_queries and d_outs:
+ * device [n_heads][dim] of io_type), which the reference's torch module
+ * converts around its calls (adaptq/torch_adapter.py:100-113): read as fp32,
+ * outputs rounded to nearest even.  A step whose tokens, the new one included,
+ * are all in the hybrid mirror (up to 512 tokens, padded 64 to 256) is one
+ * launch; any other is the step above, between conversions in the MHA's
+ * scratch memory (calls on one MHA from different streams must be ordered by
+ * the caller). */
+enum { ADAPTQ_IO_F32 = 0, ADAPTQ_IO_F16 = 1, ADAPTQ_IO_BF16 = 2 };
+int adaptq_mha_step_device(adaptq_mha_t mha, const void *d_keys, const void *d_vals,
+                           const void *d_queries, void *d_outs, int io_type,
+                           int token_pos, void *stream);
 
 /* ---- ggml operator forms ----
  * Replace the forward functions of the reference's ggml integration

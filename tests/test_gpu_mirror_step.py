@@ -1,0 +1,115 @@
+"""The decode step over the fp32 mirror in one launch, and steps whose rows are
+fp16 or bf16, against the oracle: ring bytes and scales bit-exact, outputs
+within 1e-4 norm-wise (fp32 rows); half-precision steps give the fp32 step's
+answer on the same values, rounded to nearest even, bit for bit."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from adaptq_amd import _lib
+from golden import inputs as I
+from gpu_head import GpuHead, err, rel_err, same_bits
+
+pytestmark = pytest.mark.gpu
+L = _lib.lib
+
+
+def _ptr(t):
+    return C.c_void_p(t.data_ptr())
+
+
+def _step(m, k, v, q, o, io, t):
+    n = L.adaptq_mha_step_device(m, _ptr(k), _ptr(v), _ptr(q), _ptr(o), io, t, None)
+    assert n >= 0, err()
+    return n
+
+
+# steps: tokens fed; the mirror ends past hyb tokens and at the first eviction
+@pytest.mark.parametrize("dim,kb,vb,cap,hyb,steps", [
+    (64, 4, 4, 100, 70, 110), (64, 2, 3, 600, 512, 515), (48, 3, 2, 80, 66, 70),
+    (128, 4, 2, 300, 130, 140), (80, 2, 4, 66, 512, 68), (128, 3, 16, 40, 20, 24),
+    (256, 4, 2, 80, 65, 67), (200, 16, 4, 20, 30, 24), (33, 4, 4, 20, 30, 24),
+    (512, 4, 4, 20, 10, 12), (32, 4, 4, 20, 10, 12),
+])
+def test_mirror_steps(oracle, torch_dev, dim, kb, vb, cap, hyb, steps):
+    torch = torch_dev
+    H, seed = 3, 40 + dim
+    rng = np.random.default_rng(dim + steps)
+    m = L.adaptq_mha_create(H, dim, kb, vb, cap, seed, 0.9, hyb)
+    assert m, err()
+    refs = [oracle.head(dim, kb, vb, cap, I.mha_seed(seed, h), 0.9, hyb) for h in range(H)]
+    o = torch.empty(H, dim, device="cuda")
+    for t in range(steps):
+        k, v, q = (rng.standard_normal((H, dim)).astype(np.float32) for _ in range(3))
+        if t % 7 == 3:
+            k[0] = 0.0
+            v[1] *= np.float32(1e-20)
+        kd, vd, qd = (torch.from_numpy(x).cuda() for x in (k, v, q))
+        if t == 9:
+            n = L.adaptq_mha_append_compute_all_device(m, _ptr(kd), _ptr(vd), t, _ptr(qd),
+                                                       _ptr(o), None)
+        else:
+            n = _step(m, kd, vd, qd, o, 0, t)
+        assert n == min(t + 1, cap)
+        y = o.cpu().numpy()
+        for h, r in enumerate(refs):
+            r.append(k[h], v[h], t)
+            if t < 5 or t % 16 in (0, 15) or t > steps - 6:
+                assert rel_err(y[h], r.compute(q[h])[0]) <= 1e-4, (t, h)
+    for h, r in enumerate(refs):
+        g = GpuHead.wrap(L.adaptq_mha_head(m, h), dim)
+        oi = r.info()
+        assert (g.info()["head"], g.info()["size"]) == (oi["head"], oi["size"])
+        for x, y in zip(g.read_slots(0, oi["size"]), r.read_slots(0, oi["size"])):
+            assert same_bits(x, y)
+    L.adaptq_mha_destroy(m)
+
+
+@pytest.mark.parametrize("dim,vm,hyb", [(64, 0.9, 20), (96, 0.9, 20), (64, 0.0, 0), (256, 0.0, 12)])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_half_rows(torch_dev, dim, vm, hyb, dtype):
+    """Across the mirror's end into the sparse-V and dense branches, with large
+    values and ones that underflow in the rows' type."""
+    torch = torch_dev
+    dt = getattr(torch, dtype)
+    io = {"float16": 1, "bfloat16": 2}[dtype]
+    H = 4
+    a, b = (L.adaptq_mha_create(H, dim, 4, 4, 64, 3, vm, hyb) for _ in range(2))
+    g = torch.Generator(device="cuda")
+    g.manual_seed(dim)
+    for t in range(40):
+        x = torch.randn(3, H, dim, device="cuda", generator=g)
+        x[1, 0] *= 1e-7 if t % 3 else 1e4  # (below fp16's 65,504)
+        x = x.to(dt)
+        o, o32 = torch.empty(H, dim, device="cuda", dtype=dt), torch.empty(H, dim, device="cuda")
+        x32 = x.float()
+        _step(a, x[0], x[1], x[2], o, io, t)
+        _step(b, x32[0], x32[1], x32[2], o32, 0, t)
+        assert torch.equal(o, o32.to(dt)), t
+    assert L.adaptq_mha_step_device(a, _ptr(x), _ptr(x), _ptr(x), _ptr(x), 3, 0, None) == -1
+    for m in (a, b):
+        L.adaptq_mha_destroy(m)
+
+
+def test_module_types(torch_dev):
+    """The torch module on fp32, fp16, bf16 and float64 tensors, strided ones and
+    mixed types among them: the output in q's type, as the step on fp32 values
+    gives it."""
+    torch = torch_dev
+    from adaptq_amd import AdaptQAttention
+    H, dim = 3, 64
+    base = AdaptQAttention(dim, H)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    for dt in (torch.float32, torch.float16, torch.bfloat16, torch.float64):
+        mod = AdaptQAttention(dim, H)
+        base.reset_cache()
+        for t in range(6):
+            x = torch.randn(3, 1, H, 2 * dim, device="cuda", generator=g).to(dt)
+            q, k, v = (y[..., ::2] if t % 2 else y[..., :dim] for y in x)
+            if t == 4:
+                k = k.float()
+            y = mod(q, k, v)
+            ref = base(q.float(), k.float(), v.float())
+            assert y.dtype == dt and y.shape == (1, H, dim) and torch.equal(y, ref.to(dt)), (dt, t)
