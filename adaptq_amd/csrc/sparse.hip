@@ -644,29 +644,37 @@ __device__ __forceinline__ uint32_t waves_before(const uint32_t *wsum, int wave)
   return b;
 }
 
-// Shared memory of the select kernel.  The small path (n <= kLdsSort) keeps
-// 32-bit keys, 16-bit token indices and 16 x kSelThreads 16-bit radix counts
-// (cnt also holds chain_sum_block's LDS); the large path keeps its sort keys
-// in the workspace and stages its sums' terms over the keys.
-struct SelectShared {
+// Shared memory of a selection of up to MAXN tokens.  The small path (n <=
+// kLdsSort) keeps 32-bit keys, 16-bit token indices and 16 x kSelThreads 16-bit
+// radix counts (cnt also holds the bucket counters and chain_sum_block's LDS);
+// the large path keeps its sort keys in the workspace and stages its sums'
+// terms over the keys.
+template <int MAXN>
+struct SelectSharedOf {
+  // keys; up to 4 tokens a thread the exponentials, as floats, follow the keys
+  // that the sort writes
+  static constexpr int kKeys = MAXN <= 4 * kSelThreads ? 2 * MAXN : MAXN;
+  static constexpr int kQuads = MAXN / 4 < kStage ? MAXN / 4 : kStage;
   union {
-    uint32_t key[kLdsSort];  // also the exponentials, as floats
-    float xs[seqsum_detail::kBlock * seqsum_detail::kMaxT];  // chain_sum_long's terms
+    uint32_t key[kKeys];
+    float xs[kKeys];  // chain_sum_long's terms
   };
-  uint16_t idx[kLdsSort];
-  uint16_t cnt[16 * kSelThreads];  // cnt[digit * kSelThreads + thread]
-  __align__(16) float stage[kStage];
-  float red[kSelThreads];
+  uint16_t idx[MAXN];
+  __align__(16) uint16_t cnt[16 * kSelThreads];  // cnt[digit * kSelThreads + thread]
+  __align__(16) float stage[kQuads];
+  float red[64];
   __align__(16) uint32_t wsum[kSelThreads / 64];
   float bcast[2];
   int cut;
   uint64_t last;
 };
+using SelectShared = SelectSharedOf<kLdsSort>;
 static_assert(kLdsSort == seqsum_detail::kBlock * seqsum_detail::kMaxT, "the sums' terms fit over the keys");
 
 // Block maximum with the reference's NaN-skipping compare (x > m ? x : m;
 // every partial maximum is a number, so the tree gives the sequential value).
-__device__ __forceinline__ float block_max(float m, SelectShared &sh) {
+template <class Sh>
+__device__ __forceinline__ float block_max(float m, Sh &sh) {
   for (int off = 32; off > 0; off >>= 1) {
     const float y = __shfl_xor(m, off);
     if (y > m) m = y;
@@ -685,7 +693,8 @@ __device__ __forceinline__ float block_max(float m, SelectShared &sh) {
 // the wave totals are added in order.  Counts stay packed two to a word: every
 // prefix is below 2^16 (at most 65,535 keys), so adding base * 0x10001 to a
 // word carries nothing from the low half into the high one.
-__device__ __forceinline__ void scan_counts(SelectShared &sh) {
+template <class Sh>
+__device__ __forceinline__ void scan_counts(Sh &sh) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   uint4 *c4 = reinterpret_cast<uint4 *>(sh.cnt) + 2 * tid;
   const uint4 a = c4[0], b = c4[1];
@@ -724,8 +733,8 @@ __device__ __forceinline__ void scan_counts(SelectShared &sh) {
 // give one run: a value's place in the merged run is its place in its own
 // run plus the count of smaller values in the other, found by binary search.
 // Leaves the order in sh.key[0, n) and sh.idx[0, n); touches no other key.
-template <int E>
-__device__ __forceinline__ void sort_small_merge(SelectShared &sh, int n, const uint32_t (&k)[E]) {
+template <int E, class Sh>
+__device__ __forceinline__ void sort_small_merge(Sh &sh, int n, const uint32_t (&k)[E]) {
   static_assert(E == 1 || E == 2, "one or two keys a thread");
   constexpr int NV = 2 * kSelThreads;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -809,6 +818,201 @@ __device__ __forceinline__ void sort_small_merge(SelectShared &sh, int n, const 
   __syncthreads();
 }
 
+// Bitwise OR over the wave, in lane 63: rows by DPP shifts, then across rows.
+__device__ __forceinline__ uint32_t wave_or_dpp(uint32_t v) {
+  v |= seqsum_detail::dpp_u<0x111, 0xF, 0xF, true>(v);
+  v |= seqsum_detail::dpp_u<0x112, 0xF, 0xF, true>(v);
+  v |= seqsum_detail::dpp_u<0x114, 0xF, 0xE, false>(v);
+  v |= seqsum_detail::dpp_u<0x118, 0xF, 0xC, false>(v);
+  v |= seqsum_detail::dpp_u<0x142, 0xA, 0xF, false>(v);
+  v |= seqsum_detail::dpp_u<0x143, 0xC, 0xF, false>(v);
+  return v;
+}
+
+// Stable sort of the n <= E kSelThreads keys k (thread t holds positions E t ..
+// E t + E - 1) by buckets: a bucket is a range of keys of equal length, the
+// length a power of two such that kSelThreads HB of them cover the keys' bits
+// (keys spread over at least half of the buckets, probabilities over some ten
+// octaves, a few to a bucket).  An LDS counter per bucket gives every key a
+// place in its bucket, in any order; a scan over the counters the buckets'
+// starts; a key's place in the sorted order is then its bucket's start plus the
+// keys of the bucket that are smaller, or equal and older, found by reading the
+// bucket.  (The keys of subnormal probabilities, equal steps of the value where
+// the others are steps of its logarithm, are stretched to the same scale for
+// their buckets: peaked softmaxes have many.)  Keys equal to kz, those of probabilities that are zero (peaked
+// softmaxes underflow), go last in any order: their weights are zero whichever
+// are selected.  Leaves the order in sh.key[0, n) and sh.idx[0, n) and touches
+// no other key.  Returns false, having left k alone, when a bucket holds more
+// than kBucketMax keys (ties, or keys crowded by a far outlier), which the
+// reading of buckets would pay for as much as another sort: the caller sorts
+// them otherwise.
+//
+// Bound: latency, seven barriers with a few LDS accesses between them.  Decodes
+// with it, and with the sorts before it (sort_small_merge, above 2,048 tokens a
+// radix sort of 4-bit digits): 4 heads d64 K4/V2 x 2,048 tokens 26.6 and 32.5
+// us, x 3,000 36.5 and 47.7; 8 heads x 8,192 55 and 70.5; 4 heads x 2,048 with
+// logits of +-60 (subnormal probabilities) 53.4 and 55.8.
+constexpr uint32_t kBucketMax = 512;
+
+template <int E, class Sh>
+__device__ __forceinline__ bool sort_buckets(Sh &sh, int n, const uint32_t (&k)[E],
+                                             uint32_t kz) {
+  constexpr int HB = E <= 2 ? 2 : E;  // buckets a thread
+  constexpr int NB = HB * kSelThreads;
+  constexpr int LOG_NB = HB == 2 ? 11 : HB == 4 ? 12 : 13;
+  static_assert(NB == 1 << LOG_NB && NB * 4 <= (int)sizeof(sh.cnt), "the counters fit sh.cnt");
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint32_t *hist = reinterpret_cast<uint32_t *>(sh.cnt);
+  // the key on the bucket scale: kz - k are the probability's bits
+  auto scaled = [kz](uint32_t key) -> uint32_t {
+    const uint32_t b = kz - key;
+    return b < 0x00800000u ? kz - 0x00800000u + (0x4B000000u - __float_as_uint((float)b)) : key;
+  };
+  uint32_t kor = 0u;
+#pragma unroll
+  for (int e = 0; e < E; ++e) kor |= tid * E + e < n && k[e] != kz ? scaled(k[e]) : 0u;
+  kor = wave_or_dpp(kor);
+  if (lane == 63) sh.wsum[wave] = kor;
+#pragma unroll
+  for (int j = 0; j < HB; ++j) hist[j * kSelThreads + tid] = 0u;
+  if (tid == 0) sh.cut = 0;  // zeros placed so far
+  __syncthreads();
+  kor = 0u;
+  {
+    const uint4 *w4 = reinterpret_cast<const uint4 *>(sh.wsum);
+#pragma unroll
+    for (int q = 0; q < kSelThreads / 256; ++q) {
+      const uint4 v = w4[q];
+      kor |= v.x | v.y | v.z | v.w;
+    }
+  }
+  if (kor == 0u) {  // every key is the smallest, or a zero's
+    bool zero = false;
+#pragma unroll
+    for (int e = 0; e < E; ++e) zero |= tid * E + e < n && k[e] == kz;
+    if (!__syncthreads_or(zero)) {  // all equal: the order is the tokens'
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (tid * E + e < n) {
+          sh.key[tid * E + e] = k[e];
+          sh.idx[tid * E + e] = (uint16_t)(tid * E + e);
+        }
+      __syncthreads();
+      return true;
+    }
+  }
+  const int bits = 32 - __clz((int)(kor | 1u));
+  const int sft = bits > LOG_NB ? bits - LOG_NB : 0;
+  uint32_t slot[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const bool valid = tid * E + e < n, zero = valid && k[e] == kz;
+    if (valid && !zero) slot[e] = atomicAdd(&hist[scaled(k[e]) >> sft], 1u);
+    const uint64_t zs = __ballot(zero);
+    if (zs != 0ull) {
+      int z0 = 0;
+      if (lane == 0) z0 = atomicAdd(&sh.cut, (int)__popcll(zs));
+      z0 = __builtin_amdgcn_readfirstlane(z0);
+      if (zero) slot[e] = (uint32_t)(z0 + __popcll(zs & ((1ull << lane) - 1ull)));
+    }
+  }
+  __syncthreads();
+  const int n1 = n - sh.cut;  // keys in buckets
+  // starts: thread t scans buckets HB t .. HB t + HB - 1
+  uint32_t c[HB], sum = 0u;
+  bool crowded = false;
+#pragma unroll
+  for (int j = 0; j < HB; ++j) {
+    c[j] = hist[HB * tid + j];
+    crowded |= c[j] > kBucketMax;
+    sum += c[j];
+  }
+  const uint32_t incl = seqsum_detail::wave_scan_dpp<uint32_t>(sum);
+  const bool any_crowded = __ballot(crowded) != 0ull;
+  // (the wave's total, and whether it saw a crowded bucket, in one word)
+  if (lane == 63) sh.wsum[wave] = incl | (any_crowded ? 0x80000000u : 0u);
+  __syncthreads();
+  uint32_t base = incl - sum, flags = 0u;
+  {
+    const uint4 *w4 = reinterpret_cast<const uint4 *>(sh.wsum);
+#pragma unroll
+    for (int q = 0; q < kSelThreads / 256; ++q) {
+      const uint4 v = w4[q];
+      const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        flags |= x[i];
+        base += 4 * q + i < wave ? x[i] & 0x7FFFFFFFu : 0u;
+      }
+    }
+  }
+  if (flags & 0x80000000u) {  // uniform over the block
+    __syncthreads();          // sh.wsum is read before the caller writes it
+    return false;
+  }
+#pragma unroll
+  for (int j = 0; j < HB; ++j) {
+    hist[HB * tid + j] = base;
+    base += c[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int p = tid * E + e;
+    if (p < n) {
+      const uint32_t at = k[e] == kz ? (uint32_t)n1 + slot[e] : hist[scaled(k[e]) >> sft] + slot[e];
+      sh.key[at] = k[e];
+      sh.idx[at] = (uint16_t)p;
+    }
+  }
+  __syncthreads();
+  uint32_t kk[E], ii[E], at[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int p = e * kSelThreads + tid;
+    if (p >= n1) continue;
+    kk[e] = sh.key[p];
+    ii[e] = sh.idx[p];
+    const uint32_t b = scaled(kk[e]) >> sft;
+    const uint32_t from = hist[b], to = b + 1u < (uint32_t)NB ? hist[b + 1u] : (uint32_t)n1;
+    uint32_t r = from, same = 0u;
+    for (uint32_t j = from; j < to; j += 8) {
+      uint32_t y[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) y[u] = sh.key[min(j + u, to - 1u)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        r += j + u < to && y[u] < kk[e] ? 1u : 0u;
+        same += j + u < to && y[u] == kk[e] ? 1u : 0u;
+      }
+    }
+    if (same > 1u) {  // ties, oldest first
+      for (uint32_t j = from; j < to; j += 8) {
+        uint32_t y[8], i[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const uint32_t jj = min(j + u, to - 1u);
+          y[u] = sh.key[jj];
+          i[u] = sh.idx[jj];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          r += j + u < to && y[u] == kk[e] && i[u] < ii[e] ? 1u : 0u;
+      }
+    }
+    at[e] = r;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    if (e * kSelThreads + tid >= n1) continue;
+    sh.key[at[e]] = kk[e];
+    sh.idx[at[e]] = (uint16_t)ii[e];
+  }
+  __syncthreads();
+  return true;
+}
+
 // Selection for n <= kLdsSort tokens.  Thread t owns tokens E t .. E t + E - 1
 // in registers.  Steps:
 //   1. max of the logits (the reference's start value -1e30 and compare)
@@ -816,8 +1020,8 @@ __device__ __forceinline__ void sort_small_merge(SelectShared &sh, int n, const 
 //      for bit); thread 0 adds them left to right
 //      (attention.cpp:422-426); p = e * (1/sum)
 //   3. stable sort of the 32-bit keys less the smallest one: order p
-//      descending, ties older first.  Up to 2 kSelThreads tokens:
-//      sort_small_merge (bitonic within waves, merges in LDS); above: an LSD
+//      descending, ties older first, by sort_buckets; where that declines, up
+//      to 2 kSelThreads tokens sort_small_merge (bitonic within waves, merges in LDS); above: an LSD
 //      radix sort, 4 bits a pass, in registers, skipping digits every key
 //      shares
 //   4. quad sums ((p0+p1)+p2)+p3 of the sorted order in parallel; thread 0
@@ -827,9 +1031,9 @@ __device__ __forceinline__ void sort_small_merge(SelectShared &sh, int n, const 
 //      written over the logits in token order
 //   The logits come from lg, or, with lin != null, from the caller's
 //   registers (the same tokens); the weights go to lg and, if given, to wout.
-template <int E>
+template <int E, class Sh>
 __device__ __forceinline__ void select_small(const HeadDesc *d, float v_mass, float *lg, int n, int s0,
-                             SelectShared &sh, const float *lin = nullptr,
+                             Sh &sh, const float *lin = nullptr,
                              float *wout = nullptr) {
   static_assert(E == 1 || E == 2 || E == 4 || E == 8, "tokens per thread");
   const int tid = threadIdx.x, p0 = tid * E;
@@ -856,6 +1060,7 @@ __device__ __forceinline__ void select_small(const HeadDesc *d, float v_mass, fl
   static_assert(sizeof(ChainShared) <= sizeof(sh.cnt), "chain_sum_block's LDS in sh.cnt");
   ChainShared &cs = *reinterpret_cast<ChainShared *>(sh.cnt);
   float *ef = reinterpret_cast<float *>(sh.key) + (E <= 2 ? 2048 : E == 4 ? 4096 : 0);
+  static_assert(E > 4 || sizeof(sh.key) >= (E <= 2 ? 16384 : 32768), "keys and exponentials fit");
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     ev[e] = p0 + e < n ? expf_ref(ev[e] - mx) : 0.0f;
@@ -882,6 +1087,9 @@ __device__ __forceinline__ void select_small(const HeadDesc *d, float v_mass, fl
     }
   }
   uint32_t diff = 0;
+  // (0x7F800000 - kmin: the key of a zero probability)
+  const bool sorted = sort_buckets<E>(sh, n, k, 0x7F800000u - kmin);
+  if (!sorted) {
   if constexpr (E > 2) {
     // digits every key shares do not move anything: skip their passes
     for (int off = 32; off > 0; off >>= 1) {
@@ -955,6 +1163,7 @@ __device__ __forceinline__ void select_small(const HeadDesc *d, float v_mass, fl
     sh.idx[p0 + e] = (uint16_t)ix[e];
   }
   __syncthreads();
+  }
   }
 
   // the mass loop (attention.cpp:454-472): quad sums ((p0+p1)+p2)+p3 of the
@@ -1508,8 +1717,14 @@ __device__ __forceinline__ int vcode_shift(int c) {
 }
 
 
-template <int PT, int KB, int VB, bool LOGITS_IN>
-__global__ __launch_bounds__(kSelThreads) void sparse_fused_kernel(
+// EM: the most tokens a thread (2: up to 2,048 tokens, 4: kFusedMax); OCC: the
+// least blocks a CU that the registers allow.  With the logits given, the
+// selection and the V sum take under 64 registers, so two blocks share a CU:
+// above 256 items, where a second round of blocks would follow, padded 64 runs
+// the logits kernel first too (336 heads d64 K4/V2 x 2,048 tokens: 46 us so, 59
+// in one kernel of 102 registers a block; 672 x 1,024: 55 and 68 us).
+template <int PT, int KB, int VB, bool LOGITS_IN, int EM, int OCC>
+__global__ __launch_bounds__(kSelThreads, 4 * OCC) void sparse_fused_kernel(
     HeadDesc *const *item_desc, const float *__restrict__ queries, float v_mass, float inv_sqrt_p,
     float sqrt_p, float *ws, size_t ws_stride, float *__restrict__ outs) {
   // one LDS object with the codebooks and the query first: their addresses
@@ -1525,10 +1740,10 @@ __global__ __launch_bounds__(kSelThreads) void sparse_fused_kernel(
     float cb[16];
     float2 cb2[kPairs];
     float q[PT];
-    SelectShared sel;
+    SelectSharedOf<EM * kSelThreads> sel;
   };
   __shared__ FusedShared fs;
-  SelectShared &sh = fs.sel;
+  auto &sh = fs.sel;
   float *const s_q = fs.q;
   float *const s_cb = fs.cb;
   float *const s_cbk = fs.cbk;
@@ -1553,7 +1768,7 @@ __global__ __launch_bounds__(kSelThreads) void sparse_fused_kernel(
   float *lg = ws + (size_t)item * ws_stride;
   const int s0 = (int)(((long long)d->st.head - n + cap) % cap);
   const int E = n <= kSelThreads ? 1 : n <= 2 * kSelThreads ? 2 : 4;
-  float lreg[4];  // the thread's logits when computed here
+  float lreg[EM];  // the thread's logits when computed here
   if constexpr (!LOGITS_IN) {
     // logits of the tokens select_small gives this thread (E per thread),
     // handed over in registers; the query, then their K rows and scales
@@ -1561,10 +1776,10 @@ __global__ __launch_bounds__(kSelThreads) void sparse_fused_kernel(
     // latency
     constexpr int KW = KRow<PT, KB>::words;
     const float2 qv = query_lanes(queries + (size_t)item * dim, dim, PT);
-    uint32_t kw[4][KW];
-    float ks[4];
+    uint32_t kw[EM][KW];
+    float ks[EM];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < EM; ++e) {
       const int t = tid * E + e;
       if (e < E && t < n) {
         const int slot = ring_slot(s0, t, cap);
@@ -1575,7 +1790,7 @@ __global__ __launch_bounds__(kSelThreads) void sparse_fused_kernel(
     rotate_query_exact(s_q, nullptr, dim, PT, d->signs, inv_sqrt_p, sqrt_p, &qv);
     const float attn_s = 1.0f / (sqrtf((float)dim) * (float)PT);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < EM; ++e) {
       const int t = tid * E + e;
       if (e < E && t < n) {
         kperm_raw<PT, KB>(ring_slot(s0, t, cap) & kperm_mask(PT, KB), kw[e]);
@@ -1590,7 +1805,7 @@ __global__ __launch_bounds__(kSelThreads) void sparse_fused_kernel(
   const float *lin = LOGITS_IN ? nullptr : lreg;
   if (E == 1) select_small<1>(d, v_mass, lg, n, s0, sh, lin, w_lds);
   else if (E == 2) select_small<2>(d, v_mass, lg, n, s0, sh, lin, w_lds);
-  else select_small<4>(d, v_mass, lg, n, s0, sh, lin, w_lds);
+  else if constexpr (EM == 4) select_small<4>(d, v_mass, lg, n, s0, sh, lin, w_lds);
   __syncthreads();
 
   // weighted V rows: lane (sub, u) takes unit u of token wave * TPI + sub,
@@ -1888,12 +2103,22 @@ hipError_t launch_decode_sparse(HeadDesc *const *descs, int n_items, const Decod
     if (n <= kFusedMax && (sh.padded == 64 || sh.padded == 128)) {
       // padded 128: the logits kernel's many blocks first, then the rest in
       // one block per item
+      // (with the logits given the K width is not looked at: one instance)
+      const bool pair = cnt > 256, wide = n > 2 * kSelThreads;
+#define AQ_FUSED_AS(PT, KB_, VB_, IN_, EM_, OCC_)                                                \
+  sparse_fused_kernel<PT, KB_, VB_, IN_, EM_, OCC_><<<cnt, kSelThreads, 0, s>>>(                  \
+      dsc, q, v_mass, isp, sp, w, stride, out)
 #define AQ_FUSED(PT, KB_, VB_)                                                                    \
   if (sh.padded == PT && sh.k_bits == KB_ && sh.v_bits == VB_) {                                  \
-    if (PT == 128)                                                                                \
+    if (PT == 128 || pair) {                                                                      \
       sparse_logits_kernel<PT, KB_><<<g1, kThreads, 0, s>>>(dsc, q, n, isp, sp, w, stride);        \
-    sparse_fused_kernel<PT, KB_, VB_, PT == 128><<<cnt, kSelThreads, 0, s>>>(dsc, q, v_mass, isp,  \
-                                                                              sp, w, stride, out); \
+      if (!wide) AQ_FUSED_AS(PT, 2, VB_, true, 2, 2);                                             \
+      else if (pair) AQ_FUSED_AS(PT, 2, VB_, true, 4, 2);                                         \
+      else AQ_FUSED_AS(PT, 2, VB_, true, 4, 1);                                                   \
+    } else {                                                                                      \
+      if (!wide) AQ_FUSED_AS(64, KB_, VB_, false, 2, 1);                                          \
+      else AQ_FUSED_AS(64, KB_, VB_, false, 4, 1);                                                \
+    }                                                                                             \
     const hipError_t fe = hipGetLastError();                                                      \
     if (fe != hipSuccess) return fe;                                                              \
     continue;                                                                                     \
@@ -1905,6 +2130,7 @@ hipError_t launch_decode_sparse(HeadDesc *const *descs, int n_items, const Decod
       AQ_FUSED(128, 3, 2) AQ_FUSED(128, 3, 3) AQ_FUSED(128, 3, 4)
       AQ_FUSED(128, 4, 2) AQ_FUSED(128, 4, 3) AQ_FUSED(128, 4, 4)
 #undef AQ_FUSED
+#undef AQ_FUSED_AS
     }
 #define AQ_LOGITS(PT, KB_) \
   sparse_logits_kernel<PT, KB_><<<g1, kThreads, 0, s>>>(dsc, q, n, isp, sp, w, stride)
