@@ -51,18 +51,20 @@ class AdaptQAttention(nn.Module):
             raise ValueError(f"Expected v shape {tuple(q.shape)}, got {tuple(v.shape)}.")
 
         if q.is_cuda:
-            io = _IO_TYPES.get(q.dtype, 0)
-            if k.dtype == q.dtype == v.dtype and q.dtype in _IO_TYPES:
-                qd, kd, vd = (x.detach().contiguous() for x in (q, k, v))
-            else:
-                qd, kd, vd = (x.detach().to(torch.float32).contiguous() for x in (q, k, v))
+            # a token's call is bound by the host: nothing here makes a tensor
+            # but the output's unless types differ or rows are strided
+            dtype = q.dtype
+            io = _IO_TYPES.get(dtype)
+            if io is None or k.dtype != dtype or v.dtype != dtype:
+                q, k, v = (x.detach().to(torch.float32) for x in (q, k, v))
                 io = 0
-            out = torch.empty(q.shape, dtype=qd.dtype, device=q.device)
-            self.engine._ctx.step_device(kd.data_ptr(), vd.data_ptr(), qd.data_ptr(),
-                                         out.data_ptr(), io, self.engine.pos,
-                                         torch.cuda.current_stream(q.device).cuda_stream)
-            self.engine.pos += 1
-            return out if out.dtype == q.dtype else out.to(dtype=q.dtype)
+            q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+            out = torch.empty_like(q)
+            engine = self.engine
+            engine._ctx.step_device(k.data_ptr(), v.data_ptr(), q.data_ptr(), out.data_ptr(), io,
+                                    engine.pos, torch.cuda.current_stream(q.device).cuda_stream)
+            engine.pos += 1
+            return out if out.dtype == dtype else out.to(dtype)
 
         k_np = k.detach().float().cpu().numpy()[0]
         v_np = v.detach().float().cpu().numpy()[0]
