@@ -340,6 +340,34 @@ struct DevBuf {
   }
 };
 
+// A decode's workspace.  Its size follows the split count, which is not
+// monotone in the ring's length (8 heads d128 K4/V4: 9 splits at 8,704 tokens,
+// 16 at 8,192), so a call on shorter rings can grow it while a graph captured
+// on longer ones still holds the old address.  Buffers within the splits' 8
+// MiB therefore at least double and the old ones stay until release (under 16
+// MiB in all); larger ones, of sparse-V over long rings, only grow with the
+// length and are replaced.
+struct Workspace : DevBuf {
+  static constexpr size_t kKeep = (size_t)8 << 20;
+  std::vector<void *> kept;
+  hipError_t ensure(size_t need) {
+    if (need <= bytes || !p || bytes > kKeep) return DevBuf::ensure(need);
+    void *bigger = nullptr;
+    const size_t want = std::max(need, std::min(2 * bytes, kKeep));
+    const hipError_t e = hipMalloc(&bigger, want);
+    if (e != hipSuccess) return e;
+    kept.push_back(p);
+    p = bigger;
+    bytes = want;
+    return hipSuccess;
+  }
+  void release() {
+    DevBuf::release();
+    for (void *q : kept) (void)hipFree(q);
+    kept.clear();
+  }
+};
+
 // Pinned host memory that kernels read and write directly (device-visible
 // pointer dp).  Whoever reuses or frees it first waits for the kernels that
 // may still use it.
@@ -390,7 +418,8 @@ struct Ctx {
   aq::HeadDesc **d_desc_list = nullptr;  // one entry: d_desc
   std::vector<float> stage_k, stage_v;
   int staged = 0;
-  DevBuf d_stage, d_ws, d_items;
+  DevBuf d_stage, d_items;
+  Workspace d_ws;
   PinnedBuf h_stage, h_io;  // staged rows for the append kernel; queries and outputs
   uint64_t stage_seq = 0;   // library-stream submission that last read h_stage
   int items_uploaded = 0;
@@ -404,7 +433,8 @@ struct Mha {
   DevBuf d_list;  // [n_heads] device pointers to the heads' descriptors
   DevBuf d_rep;   // [reps][n_heads] the same pointers repeated (multi-query launches)
   int rep_n = 0;  // reps held in d_rep
-  DevBuf d_ws, d_io, d_stage;
+  DevBuf d_io, d_stage;
+  Workspace d_ws;
   PinnedBuf h_stage, h_io;
   uint64_t stage_seq = 0;  // library-stream submission that last read h_stage
 };
@@ -744,7 +774,8 @@ void reset_locked(Ctx *c) {
 struct Plan {
   std::vector<Ctx *> ctxs;
   int device = 0;
-  DevBuf d_list, d_ws;
+  DevBuf d_list;
+  Workspace d_ws;
   std::mutex mu;          // one call on the plan at a time
   uint64_t seen = 0;      // epoch the cache below was read at (0: never)
   int max_n = 0;          // largest ring size

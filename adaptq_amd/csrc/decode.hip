@@ -1843,14 +1843,16 @@ SplitPlan plan_splits(int n_items, int max_n, int min_chunk, int target_blocks) 
 // Splits of the LUT kernel, by estimated time in tokens of one 512-thread
 // block alone on a CU.  A block's fixed work (query rotation, K table, merge)
 // is worth kBlock tokens (1,500 at padded 128; half with 3-bit keys, whose
-// table is a quarter of the others') and the finalize launch kFinal; two blocks on a CU run 1.16 times as fast together, each 1.72 times as
-// long while both last (1.3 assumed of the longest).  Up to 256 blocks the
-// longest decides, above it that or the sum over the CUs and an uneven end.  The estimate only ranks split counts;
-// measured (us, chosen split first): 48 items x 32,768 tokens d128 K4/V4 in 5
-// splits 58, in 6 68; 100 x 4,096 d128 K4/V2 in 2 splits 18.8, in 3 20.0; 8 x
-// 32,768 in 32 splits 19.8, in 16 24.8, in 64 21.7; 336 x 4,096 in 1 split
-// 35.0, in 2 35.3; 512 items of 256 to 6,746 tokens (log-uniform) d96 K3/V3 in
-// 3 splits 50, in 1 65.6, d128 K4/V2 in 2 splits 38, in 1 42.5.
+// table is a quarter of the others') and the finalize launch kFinal; two
+// blocks on a CU run 1.16 times as fast together, each 1.72 times as long
+// while both last (1.3 assumed of the longest).  Up to 256 blocks the longest
+// decides, above it that or the sum over the CUs and an uneven end.  The
+// estimate only ranks split counts; measured (us, chosen split first): 48
+// items x 32,768 tokens d128 K4/V4 in 5 splits 58, in 6 68; 100 x 4,096 d128
+// K4/V2 in 2 splits 18.8, in 3 20.0; 8 x 32,768 in 32 splits 19.8, in 16 24.8,
+// in 64 21.7; 336 x 4,096 in 1 split 35.0, in 2 35.3; 512 items of 256 to
+// 6,746 tokens (log-uniform) d96 K3/V3 in 3 splits 50, in 1 65.6, d128 K4/V2
+// in 2 splits 38, in 1 42.5.
 SplitPlan plan_lut(int n_items, int max_n, const DecodeShape &sh) {
   const double kBlock = (sh.k_bits == 3 ? 750.0 : 1500.0) * 128 / sh.padded;
   const double kFinal = 800.0 * 128 / sh.padded;
