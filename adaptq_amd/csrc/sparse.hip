@@ -662,7 +662,7 @@ struct SelectSharedOf {
   uint16_t idx[MAXN];
   __align__(16) uint16_t cnt[16 * kSelThreads];  // cnt[digit * kSelThreads + thread]
   __align__(16) float stage[kQuads];
-  float red[64];
+  __align__(16) float red[64];
   __align__(16) uint32_t wsum[kSelThreads / 64];
   float bcast[2];
   int cut;
@@ -839,13 +839,14 @@ __device__ __forceinline__ uint32_t wave_or_dpp(uint32_t v) {
 // keys of the bucket that are smaller, or equal and older, found by reading the
 // bucket.  (The keys of subnormal probabilities, equal steps of the value where
 // the others are steps of its logarithm, are stretched to the same scale for
-// their buckets: peaked softmaxes have many.)  Keys equal to kz, those of probabilities that are zero (peaked
-// softmaxes underflow), go last in any order: their weights are zero whichever
-// are selected.  Leaves the order in sh.key[0, n) and sh.idx[0, n) and touches
-// no other key.  Returns false, having left k alone, when a bucket holds more
-// than kBucketMax keys (ties, or keys crowded by a far outlier), which the
-// reading of buckets would pay for as much as another sort: the caller sorts
-// them otherwise.
+// their buckets: peaked softmaxes have many.)  Keys equal to kz, those of
+// probabilities that are zero (peaked softmaxes underflow), go last, oldest
+// first, each ranked by a count of the zeros before it: which of them the mass
+// takes matters where a V scale is not finite (0 times it is NaN).  Leaves the
+// order in sh.key[0, n) and sh.idx[0, n) and touches no other key.  Returns
+// false, having left k alone, when a bucket holds more than kBucketMax keys
+// (ties, or keys crowded by a far outlier), which the reading of buckets would
+// pay for as much as another sort: the caller sorts them otherwise.
 //
 // Bound: latency, seven barriers with a few LDS accesses between them.  Decodes
 // with it, and with the sorts before it (sort_small_merge, above 2,048 tokens a
@@ -868,15 +869,29 @@ __device__ __forceinline__ bool sort_buckets(Sh &sh, int n, const uint32_t (&k)[
     const uint32_t b = kz - key;
     return b < 0x00800000u ? kz - 0x00800000u + (0x4B000000u - __float_as_uint((float)b)) : key;
   };
-  uint32_t kor = 0u;
+  uint32_t kor = 0u, zeros = 0u;  // zeros: of this thread's tokens
 #pragma unroll
-  for (int e = 0; e < E; ++e) kor |= tid * E + e < n && k[e] != kz ? scaled(k[e]) : 0u;
+  for (int e = 0; e < E; ++e) {
+    const bool valid = tid * E + e < n, zero = valid && k[e] == kz;
+    kor |= valid && !zero ? scaled(k[e]) : 0u;
+    zeros += zero ? 1u : 0u;
+  }
   kor = wave_or_dpp(kor);
-  if (lane == 63) sh.wsum[wave] = kor;
+  // zeros of the wave's threads up to this one; the waves' totals in sh.red
+  uint32_t zrank = __ballot(zeros != 0u) != 0ull
+                       ? seqsum_detail::wave_scan_dpp<uint32_t>(zeros) : 0u;
+  uint32_t *zsum = reinterpret_cast<uint32_t *>(sh.red);
+  if (lane == 63) {
+    sh.wsum[wave] = kor;
+    zsum[wave] = zrank;
+  }
+  zrank -= zeros;
 #pragma unroll
   for (int j = 0; j < HB; ++j) hist[j * kSelThreads + tid] = 0u;
-  if (tid == 0) sh.cut = 0;  // zeros placed so far
   __syncthreads();
+  zrank += __builtin_amdgcn_readfirstlane(waves_before<kSelThreads / 64>(zsum, wave));
+  const int n1 = n - __builtin_amdgcn_readfirstlane(  // keys in buckets
+                         (int)waves_before<kSelThreads / 64>(zsum, kSelThreads / 64));
   kor = 0u;
   {
     const uint4 *w4 = reinterpret_cast<const uint4 *>(sh.wsum);
@@ -886,38 +901,26 @@ __device__ __forceinline__ bool sort_buckets(Sh &sh, int n, const uint32_t (&k)[
       kor |= v.x | v.y | v.z | v.w;
     }
   }
-  if (kor == 0u) {  // every key is the smallest, or a zero's
-    bool zero = false;
+  if (kor == 0u && n1 == n) {  // every key is the smallest: the order is the tokens'
 #pragma unroll
-    for (int e = 0; e < E; ++e) zero |= tid * E + e < n && k[e] == kz;
-    if (!__syncthreads_or(zero)) {  // all equal: the order is the tokens'
-#pragma unroll
-      for (int e = 0; e < E; ++e)
-        if (tid * E + e < n) {
-          sh.key[tid * E + e] = k[e];
-          sh.idx[tid * E + e] = (uint16_t)(tid * E + e);
-        }
-      __syncthreads();
-      return true;
-    }
+    for (int e = 0; e < E; ++e)
+      if (tid * E + e < n) {
+        sh.key[tid * E + e] = k[e];
+        sh.idx[tid * E + e] = (uint16_t)(tid * E + e);
+      }
+    __syncthreads();
+    return true;
   }
   const int bits = 32 - __clz((int)(kor | 1u));
   const int sft = bits > LOG_NB ? bits - LOG_NB : 0;
   uint32_t slot[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const bool valid = tid * E + e < n, zero = valid && k[e] == kz;
-    if (valid && !zero) slot[e] = atomicAdd(&hist[scaled(k[e]) >> sft], 1u);
-    const uint64_t zs = __ballot(zero);
-    if (zs != 0ull) {
-      int z0 = 0;
-      if (lane == 0) z0 = atomicAdd(&sh.cut, (int)__popcll(zs));
-      z0 = __builtin_amdgcn_readfirstlane(z0);
-      if (zero) slot[e] = (uint32_t)(z0 + __popcll(zs & ((1ull << lane) - 1ull)));
-    }
+    if (tid * E + e >= n) continue;
+    if (k[e] == kz) slot[e] = zrank++;
+    else slot[e] = atomicAdd(&hist[scaled(k[e]) >> sft], 1u);
   }
   __syncthreads();
-  const int n1 = n - sh.cut;  // keys in buckets
   // starts: thread t scans buckets HB t .. HB t + HB - 1
   uint32_t c[HB], sum = 0u;
   bool crowded = false;
