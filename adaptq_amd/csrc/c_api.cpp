@@ -24,6 +24,7 @@
 
 #include "../../include/adaptq.h"
 #include "device.hpp"
+#include "device_buffer.hpp"
 #include "launch.hpp"
 
 // Workspace of the allocation-free decode (adaptq_plan_compute_device_static):
@@ -35,6 +36,9 @@ constexpr size_t kScratchBytes = (size_t)8 << 20;
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
 namespace {
+
+using aq::DevBuf;
+using aq::KeptBuf;
 
 thread_local char tl_error[256] = "";
 
@@ -320,54 +324,6 @@ std::atomic<uint64_t> g_epoch{1};
 
 void bump_epoch() { g_epoch.fetch_add(1, std::memory_order_acq_rel); }
 
-struct DevBuf {
-  void *p = nullptr;
-  size_t bytes = 0;
-  hipError_t ensure(size_t need) {
-    if (need <= bytes) return hipSuccess;
-    if (p) (void)hipFree(p);  // hipFree waits for the device: no kernel still uses it
-    p = nullptr;
-    bytes = 0;
-    size_t want = std::max(need, (size_t)4096);
-    hipError_t e = hipMalloc(&p, want);
-    if (e == hipSuccess) bytes = want;
-    return e;
-  }
-  void release() {
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    bytes = 0;
-  }
-};
-
-// A decode's workspace.  Its size follows the split count, which is not
-// monotone in the ring's length (8 heads d128 K4/V4: 9 splits at 8,704 tokens,
-// 16 at 8,192), so a call on shorter rings can grow it while a graph captured
-// on longer ones still holds the old address.  Buffers within the splits' 8
-// MiB therefore at least double and the old ones stay until release (under 16
-// MiB in all); larger ones, of sparse-V over long rings, only grow with the
-// length and are replaced.
-struct Workspace : DevBuf {
-  static constexpr size_t kKeep = (size_t)8 << 20;
-  std::vector<void *> kept;
-  hipError_t ensure(size_t need) {
-    if (need <= bytes || !p || bytes > kKeep) return DevBuf::ensure(need);
-    void *bigger = nullptr;
-    const size_t want = std::max(need, std::min(2 * bytes, kKeep));
-    const hipError_t e = hipMalloc(&bigger, want);
-    if (e != hipSuccess) return e;
-    kept.push_back(p);
-    p = bigger;
-    bytes = want;
-    return hipSuccess;
-  }
-  void release() {
-    DevBuf::release();
-    for (void *q : kept) (void)hipFree(q);
-    kept.clear();
-  }
-};
-
 // Pinned host memory that kernels read and write directly (device-visible
 // pointer dp).  Whoever reuses or frees it first waits for the kernels that
 // may still use it.
@@ -419,7 +375,7 @@ struct Ctx {
   std::vector<float> stage_k, stage_v;
   int staged = 0;
   DevBuf d_stage, d_items;
-  Workspace d_ws;
+  KeptBuf d_ws;
   PinnedBuf h_stage, h_io;  // staged rows for the append kernel; queries and outputs
   uint64_t stage_seq = 0;   // library-stream submission that last read h_stage
   int items_uploaded = 0;
@@ -431,10 +387,13 @@ struct Mha {
   int device = 0;
   std::mutex mu;  // whole-MHA calls; taken before any head's lock
   DevBuf d_list;  // [n_heads] device pointers to the heads' descriptors
-  DevBuf d_rep;   // [reps][n_heads] the same pointers repeated (multi-query launches)
+  // [reps][n_heads] the same pointers repeated (multi-query launches).  Entry i
+  // is head i % n_heads's for any reps: writing a list for another count leaves
+  // the entries that a graph reads as they were
+  KeptBuf d_rep;
   int rep_n = 0;  // reps held in d_rep
-  DevBuf d_io, d_stage;
-  Workspace d_ws;
+  DevBuf d_stage;
+  KeptBuf d_io, d_ws;
   PinnedBuf h_stage, h_io;
   uint64_t stage_seq = 0;  // library-stream submission that last read h_stage
 };
@@ -775,7 +734,7 @@ struct Plan {
   std::vector<Ctx *> ctxs;
   int device = 0;
   DevBuf d_list;
-  Workspace d_ws;
+  KeptBuf d_ws;
   std::mutex mu;          // one call on the plan at a time
   uint64_t seen = 0;      // epoch the cache below was read at (0: never)
   int max_n = 0;          // largest ring size

@@ -62,3 +62,55 @@ def test_captured_workspace(torch_dev, heads, dim, full, short, whole_mha):
     del graph
     L.adaptq_plan_destroy(p)
     L.adaptq_mha_destroy(m)
+
+
+@pytest.mark.parametrize("pad", [0, 8])
+def test_captured_many_queries(torch_dev, pad):
+    """The same for the many-query kernels' partials (64 queries: 15.7 MB at
+    8,300 tokens, 17.3 MB at 8,192), a larger query count (a longer descriptor
+    list) and, with padded rows, the operator's copies of them.  That the old
+    buffers are still allocated is seen from the free memory before the graph
+    runs again."""
+    torch = torch_dev
+    heads, dim, full, short, nq = 8, 128, 8300, 8192, 64
+    g = torch.Generator(device="cuda").manual_seed(pad)
+    k, v = (torch.randn(heads, full, dim, generator=g, device="cuda") for _ in range(2))
+    q = torch.randn(2 * nq, heads, dim + pad, generator=g, device="cuda")
+    m = L.adaptq_mha_create(heads, dim, 4, 4, full, 42, 0.0, 0)
+    assert m, err()
+    rows = {n: (k[:, :n].contiguous(), v[:, :n].contiguous()) for n in (full, short)}
+
+    def fill(n):
+        assert L.adaptq_mha_append_all_device(m, *map(_ptr, rows[n]), n, 0, None) == 0, err()
+        torch.cuda.synchronize()
+
+    def decode(out, n_queries, stream=None):
+        row = 4 * (dim + pad)
+        return L.adaptq_ggml_attn_f32_device(m, _ptr(q), dim, heads, n_queries, row, heads * row,
+                                             _ptr(out), row, heads * row, stream) >= 0
+
+    want, got, other = (torch.zeros_like(q) for _ in range(3))
+    fill(full)
+    assert decode(want, nq), err()
+    torch.cuda.synchronize()
+    s, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        ok = decode(got, nq, C.c_void_p(s.cuda_stream))
+    assert ok, err()
+    for count in (nq, 2 * nq):
+        L.adaptq_mha_reset(m)
+        fill(short)
+        before = torch.cuda.mem_get_info()[0]
+        assert decode(other, count), err()
+        torch.cuda.synchronize()
+        # the new workspace alone takes over 16 MB, if no old one was freed for it
+        if count == nq:
+            assert before - torch.cuda.mem_get_info()[0] >= 16 << 20
+        L.adaptq_mha_reset(m)
+        fill(full)
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got[:nq], want[:nq]) and not got[nq:].any()
+    del graph
+    L.adaptq_mha_destroy(m)
