@@ -386,7 +386,9 @@ struct Mha {
   int n_heads = 0;
   int device = 0;
   std::mutex mu;  // whole-MHA calls; taken before any head's lock
-  DevBuf d_list;  // [n_heads] device pointers to the heads' descriptors
+  // [n_heads] device pointers to the heads' descriptors, then a step's four rows
+  // of [n_heads][dim] floats (see step_rows_at)
+  DevBuf d_list;
   // [reps][n_heads] the same pointers repeated (multi-query launches).  Entry i
   // is head i % n_heads's for any reps: writing a list for another count leaves
   // the entries that a graph reads as they were
@@ -399,6 +401,16 @@ struct Mha {
 };
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+// The fp32 rows (keys, values, queries, outputs: i of 4) of a step whose caller's
+// rows are not fp32.  They are made with the MHA, so that a step allocates
+// nothing for them (it may be captured) and no other call moves them.
+size_t step_row_bytes(const Mha *m) { return align256(4 * (size_t)m->n_heads * m->heads[0]->dim); }
+float *step_rows_at(const Mha *m, int i) {
+  return reinterpret_cast<float *>(static_cast<uint8_t *>(m->d_list.p) +
+                                   align256(sizeof(void *) * (size_t)m->n_heads) +
+                                   i * step_row_bytes(m));
+}
 
 // Whether appending n tokens to these contexts copies any to a hybrid mirror
 // (from the host's ring states; it picks the append's launch shape only).
@@ -1004,18 +1016,13 @@ int step_device(Mha *m, const void *dk, const void *dv, const void *dq, void *do
     const float *q = static_cast<const float *>(dq);
     float *o = static_cast<float *>(dout);
     if (io != aq::IoType::F32) {
-      const size_t each = align256(count * 4);
-      if (hip_fail(m->d_io.ensure(4 * each), fn)) return -1;
-      auto at = [&](int i) {
-        return reinterpret_cast<float *>(static_cast<uint8_t *>(m->d_io.p) + i * each);
-      };
-      float *const dst[3] = {at(0), at(1), at(2)};
+      float *const dst[3] = {step_rows_at(m, 0), step_rows_at(m, 1), step_rows_at(m, 2)};
       const void *const src[3] = {dk, dv, dq};
       if (hip_fail(aq::launch_to_f32(dst, src, 3, count, io, s), fn)) return -1;
       k = dst[0];
       v = dst[1];
       q = dst[2];
-      o = at(3);
+      o = step_rows_at(m, 3);
     }
     n = step_all_locked(m, k, v, q, o, s, fn);
     if (n == -2) {  // the append and the decode as two launches
@@ -1145,7 +1152,9 @@ adaptq_mha_t adaptq_mha_create(int n_heads, int dim, int k_bits, int v_bits, int
   for (int i = 0; i < n_heads; ++i) list[i] = m->heads[i]->d_desc;
   {
     DeviceGuard g(m->device);
-    if (hip_fail(m->d_list.ensure(sizeof(void *) * (size_t)n_heads), "adaptq_mha_create") ||
+    if (hip_fail(m->d_list.ensure(align256(sizeof(void *) * (size_t)n_heads) +
+                                  4 * step_row_bytes(m)),
+                 "adaptq_mha_create") ||
         hip_fail(hipMemcpy(m->d_list.p, list.data(), sizeof(void *) * n_heads,
                            hipMemcpyHostToDevice),
                  "adaptq_mha_create")) {

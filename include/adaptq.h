@@ -206,9 +206,9 @@ int adaptq_mha_append_compute_all_device(adaptq_mha_t mha, const float *d_keys,
  * converts around its calls (adaptq/torch_adapter.py:100-113): read as fp32,
  * outputs rounded to nearest even.  A step whose tokens, the new one included,
  * are all in the hybrid mirror (up to 512 tokens, padded 64 to 256) is one
- * launch; any other is the step above, between conversions in the MHA's
- * scratch memory (calls on one MHA from different streams must be ordered by
- * the caller). */
+ * launch; any other is the step above, between conversions in memory that the
+ * MHA holds for them from its creation (calls on one MHA from different streams
+ * must be ordered by the caller). */
 enum { ADAPTQ_IO_F32 = 0, ADAPTQ_IO_F16 = 1, ADAPTQ_IO_BF16 = 2 };
 int adaptq_mha_step_device(adaptq_mha_t mha, const void *d_keys, const void *d_vals,
                            const void *d_queries, void *d_outs, int io_type,

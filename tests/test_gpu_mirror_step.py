@@ -113,3 +113,43 @@ def test_module_types(torch_dev):
             y = mod(q, k, v)
             ref = base(q.float(), k.float(), v.float())
             assert y.dtype == dt and y.shape == (1, H, dim) and torch.equal(y, ref.to(dt)), (dt, t)
+
+
+@pytest.mark.parametrize("dim,vm,hyb", [(64, 0.0, 0), (128, 0.0, 0), (64, 0.9, 20)])
+def test_half_rows_captured_first(torch_dev, dim, vm, hyb):
+    """A half-precision step that no such step went before, captured: its
+    conversions take no memory that is not there, and later calls on the MHA (the
+    ggml operator's, on more and strided rows) leave that memory to the graph."""
+    torch = torch_dev
+    H, n, nq = 4, 20, 40
+    a, b = (L.adaptq_mha_create(H, dim, 4, 4, 64, 3, vm, hyb) for _ in range(2))
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    rows = torch.randn(2, H, n, dim, device="cuda", generator=g)
+    x = torch.randn(3, H, dim, device="cuda", generator=g).half()
+    for m in (a, b):
+        assert L.adaptq_mha_append_all_device(m, _ptr(rows[0]), _ptr(rows[1]), n, 0, None) == 0
+    torch.cuda.synchronize()
+    want, got = (torch.zeros(H, dim, device="cuda", dtype=torch.float16) for _ in range(2))
+    if vm:  # sparse-V needs a workspace: any decode of this branch leaves one
+        for m in (a, b):
+            f = x.float()
+            _step(m, f[0], f[1], f[2], torch.empty_like(f[0]), 0, n)
+        torch.cuda.synchronize()
+    s, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        r = L.adaptq_mha_step_device(a, _ptr(x[0]), _ptr(x[1]), _ptr(x[2]), _ptr(got), 1, n,
+                                     C.c_void_p(s.cuda_stream))
+    assert r > 0, err()
+    q = torch.randn(nq, H, dim + 8, device="cuda", generator=g)
+    o, row = torch.empty_like(q), 4 * (dim + 8)
+    for m in (a, b):
+        assert L.adaptq_ggml_attn_f32_device(m, _ptr(q), dim, H, nq, row, H * row, _ptr(o), row,
+                                             H * row, None) >= 0, err()
+    torch.cuda.synchronize()
+    graph.replay()
+    _step(b, x[0], x[1], x[2], want, 1, n)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    del graph
+    for m in (a, b):
+        L.adaptq_mha_destroy(m)
