@@ -402,6 +402,12 @@ struct Mha {
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// Whether two ranges of n bytes are the very same or do not overlap.
+bool apart_or_same(const void *a, const void *b, size_t n) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x == y || x + n <= y || y + n <= x;
+}
+
 // The fp32 rows (keys, values, queries, outputs: i of 4) of a step whose caller's
 // rows are not fp32.  They are made with the MHA, so that a step allocates
 // nothing for them (it may be captured) and no other call moves them.
@@ -976,13 +982,17 @@ int step_all_locked(Mha *m, const float *dk, const float *dv, const float *dq, f
 
 // The same on the hybrid branch, in one launch (launch_mirror_step), for rows
 // of any IoType: when every head's mirror holds the same tokens, all of its
-// ring, after the append.  Returns -2, having launched nothing, when it does
-// not; the common ring size, or -1.
+// ring, after the append, and the outputs lie apart from the keys and values or
+// exactly on them (a head's rows are read before its output is written, other
+// heads' may not be; the append launch of the two-launch step reads them all).
+// Returns -2, having launched nothing, when not so; the common ring size, or -1.
 int mirror_step_locked(Mha *m, const void *dk, const void *dv, const void *dq, void *dout,
                        aq::IoType io, hipStream_t s, const char *fn) {
   const Ctx *c0 = m->heads[0];
   const aq::RingState a0 = aq::ring_after(c0->st, 1, c0->cap, c0->hyb);
   if (!aq::mirror_step_supported(m->n_heads, c0->padded, a0.size)) return -2;
+  const size_t bytes = (size_t)m->n_heads * c0->dim * (io == aq::IoType::F32 ? 4 : 2);
+  if (!apart_or_same(dk, dout, bytes) || !apart_or_same(dv, dout, bytes)) return -2;
   for (const Ctx *c : m->heads) {
     const aq::RingState a = aq::ring_after(c->st, 1, c->cap, c->hyb);
     if (c->staged != 0 || a.size != a0.size || mode_at(c, a) != Mode::Hybrid) return -2;
@@ -1644,9 +1654,8 @@ int adaptq_ggml_attn_f32_device(adaptq_mha_t h, const float *d_q, int head_dim, 
     return (H == 1 || nb1 == (size_t)head_dim * 4) &&
            (n_queries == 1 || nb2 == (size_t)H * head_dim * 4);
   };
-  const uintptr_t qa = reinterpret_cast<uintptr_t>(d_q), da = reinterpret_cast<uintptr_t>(d_dst);
-  const bool direct = packed(q_nb1, q_nb2) && packed(d_nb1, d_nb2) &&
-                      (qa == da || qa + bytes <= da || da + bytes <= qa);
+  const bool direct =
+      packed(q_nb1, q_nb2) && packed(d_nb1, d_nb2) && apart_or_same(d_q, d_dst, bytes);
   const float *dq = d_q;
   float *dout = d_dst;
   if (hip_fail(caller_begin(m->device, s), fn)) return -1;

@@ -153,3 +153,32 @@ def test_half_rows_captured_first(torch_dev, dim, vm, hyb):
     del graph
     for m in (a, b):
         L.adaptq_mha_destroy(m)
+
+
+@pytest.mark.parametrize("place", ["keys", "vals", "same keys", "same vals", "same queries"])
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+def test_outputs_over_rows(torch_dev, place, dtype):
+    """Outputs shifted into the step's keys or values (more heads than run at
+    once, so that some would read rows that others have written over) or exactly on
+    its rows."""
+    torch = torch_dev
+    dt, io = getattr(torch, dtype), 0 if dtype == "float32" else 1
+    # (a multiple of 8 heads on: the same XCD, whose L2 shows it the writes)
+    H, dim, shift = 2048, 64, 1504
+    g = torch.Generator(device="cuda").manual_seed(3)
+    first, x = (torch.randn(3, H, dim, device="cuda", generator=g).to(dt) for _ in range(2))
+    want = torch.empty(H, dim, device="cuda", dtype=dt)
+    at = ("keys", "vals", "queries").index(place.split()[-1])
+    off = 0 if place.startswith("same") else shift * dim
+    bufs = [torch.zeros(H + shift, dim, device="cuda", dtype=dt) for _ in range(3)]
+    for b, r in zip(bufs, x):
+        b[:H] = r
+    out = bufs[at].view(-1)[off:off + H * dim]
+    for rows, o in ((x, want), (bufs, out)):
+        m = L.adaptq_mha_create(H, dim, 4, 4, 8, 5, 0.0, 8)
+        assert m, err()
+        _step(m, *first, torch.empty_like(want), io, 0)
+        _step(m, *rows, o, io, 1)
+        torch.cuda.synchronize()
+        L.adaptq_mha_destroy(m)
+    assert torch.equal(out.view(H, dim), want)
