@@ -51,7 +51,9 @@ __global__ __launch_bounds__(kStepThreads) void mirror_step_kernel(
   HeadDesc *d = item_desc[item];
   const RingState st = d->st;
   const int n0 = __builtin_amdgcn_readfirstlane(st.raw_count);  // mirror rows before the step
-  const int n = n0 + 1;
+  // (the host plans at most kMaxTokens; a captured step's ring goes on growing with
+  // the replays, which attend over the oldest kMaxTokens from then on)
+  const int n = min(n0 + 1, kMaxTokens);
   const float *raw_k = d->raw_k, *raw_v = d->raw_v;
   // the step's rows and query as fp32 in LDS, zeros past dim
   const size_t row0 = (size_t)item * dim;

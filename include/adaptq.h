@@ -177,7 +177,22 @@ int adaptq_mha_compute_all(adaptq_mha_t mha, const float *queries, float *outs);
  * returns the ring size, or -1 (also when the heads differ in ring size or
  * branch, e.g. after per-head appends: use adaptq_mha_compute_all then).
  * Host inspection calls (read_slots, ring_info) see device-path appends once
- * the caller's stream has been synchronised. */
+ * the caller's stream has been synchronised.
+ *
+ * HIP graphs.  The device forms of decodes, appends and steps (of an MHA, a plan
+ * or the ggml operators) may be captured, adaptq_plan_compute_device_static
+ * excepted.  A reset or host-form call shortly before needs an inspection call
+ * (adaptq_read_slots) in between, which waits for it.  A replay works on the rings
+ * as they are then, with the launches planned for the branch and the ring sizes at
+ * capture; rings must be no longer than that (a longer one is attended over in
+ * part, and under sparse-V the workspace is too small for it).  A captured append
+ * advances the host's view of the rings once, at capture.  Nothing is allocated or
+ * uploaded under capture: a call that needs more workspace, or another query count
+ * of the ggml operator, than an earlier call on the same plan or MHA fails, unless
+ * one block a context can do it (a dense decode of one query a head at padded 64
+ * to 256).  What a decode or a step uses stays allocated until its plan or MHA is
+ * destroyed; the ggml append's copy of its rows may move when a later one is
+ * larger. */
 int adaptq_mha_append_all_device(adaptq_mha_t mha, const float *d_keys,
                                  const float *d_vals, int n_tokens,
                                  int first_pos, void *stream);

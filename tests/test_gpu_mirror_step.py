@@ -182,3 +182,32 @@ def test_outputs_over_rows(torch_dev, place, dtype):
         torch.cuda.synchronize()
         L.adaptq_mha_destroy(m)
     assert torch.equal(out.view(H, dim), want)
+
+
+def test_captured_step_past_the_kernel(torch_dev):
+    """A step captured at 510 tokens and replayed past the 512 that its launch
+    covers: those 512, the oldest, keep their softmax."""
+    torch = torch_dev
+    H, dim, n, replays = 3, 64, 509, 12
+    g = torch.Generator(device="cuda").manual_seed(8)
+    rows = torch.randn(2, H, n, dim, device="cuda", generator=g)
+    x = torch.randn(3, H, dim, device="cuda", generator=g)
+    out = torch.zeros(H, dim, device="cuda")
+    m = L.adaptq_mha_create(H, dim, 4, 4, 1000, 3, 0.0, 600)
+    assert L.adaptq_mha_append_all_device(m, _ptr(rows[0]), _ptr(rows[1]), n, 0, None) == 0, err()
+    torch.cuda.synchronize()
+    s, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        r = L.adaptq_mha_step_device(m, _ptr(x[0]), _ptr(x[1]), _ptr(x[2]), _ptr(out), 0, n,
+                                     C.c_void_p(s.cuda_stream))
+    assert r == n + 1, err()
+    for i in range(1, replays + 1):
+        graph.replay()
+        torch.cuda.synchronize()
+        c = min(i, 512 - n)
+        k, v = (torch.cat((old, new[:, None].expand(H, c, dim)), 1).double().cpu()
+                for old, new in ((rows[0], x[0]), (rows[1], x[1])))
+        w = torch.softmax((k * x[2].double().cpu()[:, None]).sum(2) / dim ** 0.5, 1)
+        assert rel_err(out.cpu(), (w[:, :, None] * v).sum(1)) <= 1e-5, i
+    del graph
+    L.adaptq_mha_destroy(m)
