@@ -7,13 +7,15 @@
                                    compiled with AQ_CLOCK_STAMPS (per-block
                                    shader-clock stamps of the LUT decode kernel,
                                    read by ``bench.py --clock-stamps``)
-  adaptq_amd/libadaptq_probe.so    timing library: the bulk append's memory
-                                   traffic without its codec (probe_rows.hip,
-                                   read by ``bench.py --append-floor``)
+  adaptq_amd/libadaptq_probe.so    probes: the bulk append's memory traffic
+                                   without its codec (probe_rows.hip, read by
+                                   ``bench.py --append-floor``) and the matrix
+                                   cores' fp32 chain against fmaf
+                                   (probe_chain.hip, read by a test)
 
 Run ``python -m adaptq_amd.build`` or call :func:`build` (all four).  Every
-call recompiles.  ``--clock-stamps`` or ``--probes`` builds only that timing
-library.  The product never loads the timing libraries.
+call recompiles.  ``--clock-stamps`` or ``--probes`` builds only that library.
+The product never loads these two.
 """
 from __future__ import annotations
 
@@ -47,6 +49,7 @@ HIP_FLAGS = [
 
 SOURCES = ["append.hip", "decode.hip", "mirror_step.hip", "mquery.hip", "sparse.hip", "layout.hip",
            "kbackend.hip", "c_api.cpp", "vtable.cpp"]
+PROBE_SOURCES = ["probe_rows.hip", "probe_chain.hip"]
 
 
 def _run(cmd):
@@ -95,12 +98,15 @@ def build_clock_lib() -> str:
 
 def build_probe_lib() -> str:
     """libadaptq_probe.so: the bulk append's memory traffic without its codec
-    (probe_rows.hip; bench.py --append-floor)."""
+    (probe_rows.hip; bench.py --append-floor) and the fp32 chain of the matrix
+    cores (probe_chain.hip)."""
     os.makedirs(BUILD, exist_ok=True)
-    obj = os.path.join(BUILD, "probe_rows.hip.o")
-    _run([HIPCC, *HIP_FLAGS, "-x", "hip", "-c", os.path.join(CSRC, "probe_rows.hip"), "-o", obj])
+    objs = []
+    for src in PROBE_SOURCES:
+        objs.append(os.path.join(BUILD, src + ".o"))
+        _run([HIPCC, *HIP_FLAGS, "-x", "hip", "-c", os.path.join(CSRC, src), "-o", objs[-1]])
     tmp = PROBE_LIB + ".tmp"
-    _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", obj, "-o", tmp,
+    _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp,
           f"-Wl,-rpath,{ROCM}/lib", "-Wl,-soname,libadaptq_probe.so"])
     os.replace(tmp, PROBE_LIB)
     return PROBE_LIB
@@ -122,7 +128,7 @@ def build_pybind() -> str:
 
 
 def build(jobs: int = 8) -> None:
-    """The library, its Python module and the two timing libraries."""
+    """The library, its Python module, the timing library and the probes."""
     build_lib(jobs)
     build_pybind()
     build_clock_lib()

@@ -19,8 +19,8 @@
 //
 // Both products run on the matrix cores.  v_mfma_f32_16x16x4 adds its four
 // products to an entry one after another, in order, each a fused multiply-add
-// rounded as fmaf (checked on the device against fmaf, bit for bit, over
-// normal, denormal and large operands), so a chain of it is a chain of the
+// rounded as fmaf (tests/test_gpu_mfma_chain.py: bit for bit, over normal,
+// denormal and large operands), so a chain of it is a chain of the
 // reference's: eight accumulators, chain L of a 16-token by 16-query tile fed
 // dims L + 8 j, j ascending, four an instruction.  Operand layouts
 // (established on the device): lane l supplies A[l % 16][l / 16] and
