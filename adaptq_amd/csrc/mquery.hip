@@ -60,6 +60,7 @@
 #include <algorithm>
 
 #include "launch.hpp"
+#include "mquery_rule.hpp"
 
 namespace aq {
 
@@ -67,10 +68,7 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kMqWaves = 4;
 constexpr int kMqThreads = 64 * kMqWaves;
-constexpr int kMqQueries = 16;  // queries per wave
-constexpr int kMqTile = 16;     // tokens per wave step
 constexpr float kLog2e = 1.44269504088896340736f;
 
 // The codes of dims 8 j .. 8 j + 7 of a packed row (MSB-first,
@@ -477,57 +475,12 @@ __global__ __launch_bounds__(kMqThreads, QG == 4 ? 3 : 2) void decode_mq_kernel(
   }
 }
 
-struct MqPlan {
-  int splits, chunk, qgroups;
-  int qg;       // query groups a block
-  int qblocks;  // blocks over the query groups
-};
-
-MqPlan mq_plan(int n_heads, int nq, int max_n) {
-  MqPlan mp;
-  mp.qgroups = (nq + kMqQueries - 1) / kMqQueries;
-  mp.qg = mp.qgroups >= 3 ? 4 : mp.qgroups;
-  mp.qblocks = (mp.qgroups + mp.qg - 1) / mp.qg;
-  const int max1 = max_n > 0 ? max_n : 1;
-  // two blocks a CU (256 CUs), of at least 128 tokens each.  Measured, 64
-  // queries of 8 heads d128 K4/V4 x 32,768 tokens, the whole call: one block a
-  // CU 147 us, two 129, three (as many as the registers allow) 130 with half
-  // as much finalize work again.
-  const int step = kMqTile * (kMqWaves / mp.qg);
-  const int blocks = n_heads * mp.qblocks;
-  const int splits = std::max(1, std::min(512 / blocks, (max1 + 127) / 128));
-  int chunk = (max1 + splits - 1) / splits;
-  chunk = ((chunk + step - 1) / step) * step;
-  mp.chunk = chunk;
-  mp.splits = (max1 + chunk - 1) / chunk;
-  return mp;
-}
-
-// Whether the matrix-core kernel takes nq queries of n_heads heads over max_n
-// tokens, rather than the LUT kernel as nq * n_heads items.  The LUT kernel
-// pays for each query, about 4.5 M values of K a microsecond, in one launch
-// or two; this one for groups of 16 queries, about 11 M values a microsecond,
-// and 10 us more for its rotation and finalize launches.  Measured (whole
-// call, LUT and matrix cores): 8 heads d128 K4/V4 x 32,768 tokens, 4 queries
-// 41 and 51 us, 8 queries 68 and 51, 12 queries 116 and 52; 16 heads d64 K4/V2
-// x 16,384, 8 queries 26 and 31, 12 queries 36 and 32; 2 heads d128 K3/V3 x
-// 32,768, 12 queries 39 and 38; 12 heads d128 x 512, 12 queries 9 and 18; 4
-// heads d64 x 1,024, 12 queries 7 and 14.
-constexpr int kMqMinQueries = 8;
-
-bool mq_pays(int n_heads, int nq, const DecodeShape &sh) {
-  if (nq < kMqMinQueries) return false;
-  const double per_query = (double)n_heads * (sh.max_n > 0 ? sh.max_n : 1) * sh.padded;
-  const int padded_nq = (nq + kMqQueries - 1) / kMqQueries * kMqQueries;
-  return nq * per_query / 4.5e6 > 10.0 + padded_nq * per_query / 1.1e7;
-}
-
 bool mq_eligible(int n_items, int n_heads, const DecodeShape &sh) {
   if (n_heads <= 0 || n_items % n_heads != 0) return false;
   const int nq = n_items / n_heads;
   const bool kq = sh.k_bits >= 2 && sh.k_bits <= 4, vq = sh.v_bits >= 2 && sh.v_bits <= 4;
   return !sh.raw && kq && vq && (sh.padded == 64 || sh.padded == 128) &&
-         mq_pays(n_heads, nq, sh) && n_heads <= 65535 && (int64_t)n_heads * ((nq + kMqQueries - 1) / kMqQueries) *
+         mq_pays(n_heads, nq, sh.max_n, sh.padded) && n_heads <= 65535 && (int64_t)n_heads * ((nq + kMqQueries - 1) / kMqQueries) *
                                       ((sh.max_n + 127) / 128) <
                                   (int64_t)1 << 31;
 }
@@ -558,7 +511,7 @@ hipError_t dispatch_mq(const DecodeShape &sh, dim3 grid, HeadDesc *const *descs,
 }
 
 // Workspace of the multi-query path: the rotated queries (n_heads * qgroups
-// * 64 rows of P floats), then the split partials (item, split) of P + 4.
+// * 16 rows of P floats), then the split partials (item, split) of P + 4.
 size_t mq_qrot_floats(int n_heads, const MqPlan &mp, int padded) {
   return (size_t)n_heads * mp.qgroups * kMqQueries * padded;
 }

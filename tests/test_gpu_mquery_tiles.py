@@ -1,13 +1,14 @@
 """The many-query kernel at the edges of its tiles (16 tokens, 16 queries a
 wave, 1, 2 or 4 query groups a block, slices of a step, splits over tokens)
-and of the rule that takes it, against the oracle: within 1e-4 norm-wise, as
-every output test; the logits repeat the reference's own fp32 steps, so plain
-N(0,1) rings stay far below."""
+and of the rule that takes it (7 queries: the LUT kernel), against the oracle:
+within 1e-4 norm-wise, as every output test; the logits repeat the reference's
+own fp32 steps, so plain N(0,1) rings stay far below."""
 import ctypes as C
 
 import numpy as np
 import pytest
 
+import mq_rule
 from adaptq_amd import _lib
 from golden import inputs as I
 from gpu_head import err, rel_err
@@ -20,20 +21,23 @@ L = _lib.lib
                                        (48, 3, 2), (64, 2, 4)])
 @pytest.mark.parametrize("nq", [7, 8, 16, 17, 32, 33, 49, 64, 65])
 def test_tile_edges(oracle, torch_dev, dim, kb, vb, nq):
-    """Enough heads that the kernel takes the call (from 8 queries on); rings of
-    whole tiles, one token more or less, a whole and a part step or split, and
+    """As many heads as the kernel takes the call at (from 8 queries on); rings
+    of whole tiles, one token more or less, a whole and a part step or split, and
     a wrapped one."""
     torch = torch_dev
     rng = np.random.default_rng(dim + 10 * kb + nq)
-    H, cap, seed = 96, 1300, 11 * dim + nq
+    sizes, cap, seed = (1023, 1024, 1025, 1037, 1281, 1500), 1300, 11 * dim + nq
+    P = 64 if dim <= 64 else 128
+    H = mq_rule.heads_for(nq, sizes[0], P) if nq >= 8 else 96
+    assert all(mq_rule.takes(H, nq, min(n, cap), P) == (nq >= 8) for n in sizes)
     m = L.adaptq_mha_create(H, dim, kb, vb, cap, seed, 0.0, 0)
     assert m, err()
-    check = (0, 61, H - 1)
+    check = (0, H // 2, H - 1)
     refs = {h: oracle.head(dim, kb, vb, cap, I.mha_seed(seed, h)) for h in check}
     qd = torch.from_numpy((rng.standard_normal((nq, H, dim)) * 2).astype(np.float32)).cuda()
     qs, od, row = qd.cpu().numpy(), torch.empty_like(qd), 4 * dim
     done = 0
-    for n in (1023, 1024, 1025, 1037, 1281, 1500):
+    for n in sizes:
         kd, vd = (torch.from_numpy(rng.standard_normal((H, n - done, dim)).astype(np.float32)).cuda()
                   for _ in range(2))
         assert L.adaptq_mha_append_all_device(m, C.c_void_p(kd.data_ptr()),
