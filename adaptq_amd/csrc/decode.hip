@@ -2112,16 +2112,16 @@ hipError_t launch_decode_items(HeadDesc *const *descs, int n_items, const Decode
     // splits fastest a split count that shares a factor with 8 puts the last
     // splits of every item (empty ones, where rings differ in length) on the
     // same XCDs and the first ones on the others
-    const dim3 grid(n_items, sp.splits);
+    const dim3 items_first(n_items, sp.splits);
     if (sh.padded == 64)
-      e = raw ? dispatch_lut<64, true>(sh, grid, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s)
-              : dispatch_lut<64, false>(sh, grid, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s);
+      e = raw ? dispatch_lut<64, true>(sh, items_first, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s)
+              : dispatch_lut<64, false>(sh, items_first, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s);
     else if (sh.padded == 256)
-      e = raw ? dispatch_lut<256, true>(sh, grid, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s)
-              : dispatch_lut<256, false>(sh, grid, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s);
+      e = raw ? dispatch_lut<256, true>(sh, items_first, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s)
+              : dispatch_lut<256, false>(sh, items_first, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s);
     else
-      e = raw ? dispatch_lut<128, true>(sh, grid, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s)
-              : dispatch_lut<128, false>(sh, grid, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s);
+      e = raw ? dispatch_lut<128, true>(sh, items_first, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s)
+              : dispatch_lut<128, false>(sh, items_first, descs, d_q, sp.chunk, sp.splits, d_ws, d_out, s);
     if (e != hipSuccess || sp.splits == 1) return e;  // one split: the kernel finished the items
   } else if (wide_eligible(sh)) {
     e = sh.padded == 512 ? dispatch_wide<512>(sh, grid, descs, d_q, sp.chunk, sp.splits, d_ws, s)

@@ -20,7 +20,7 @@
 //
 // Kernels: one grid over (token blocks, items) computes the logits and the
 // blocks' maxima.  Up to 8,192 tokens, one block per item then does softmax,
-// the sort (a stable radix sort in LDS) and the cut, and turns the selection
+// the sort (stable, in LDS) and the cut, and turns the selection
 // into per-token weights.  Above, a grid computes the exponentials, one block
 // per item their left-to-right sum and the sort keys, a per-item radix sort
 // over many blocks orders them, and one block per item takes the cut.  A grid over
@@ -42,7 +42,7 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kSelThreads = 1024;
 // Rings up to kSelectInBlock tokens are selected inside the select kernel
-// (radix sort in LDS); longer ones sort over many blocks between two kernels
+// (sorted in LDS); longer ones sort over many blocks between two kernels
 // (measured, 8 heads d128: 12,000 tokens 242 -> 198 us and 16,384 tokens
 // 264 -> 237 us sorted outside the select kernel; at 8,192 tokens and below
 // the in-block sort is as fast or faster).
@@ -1020,15 +1020,15 @@ __device__ __forceinline__ bool sort_buckets(Sh &sh, int n, const uint32_t (&k)[
 // in registers.  Steps:
 //   1. max of the logits (the reference's start value -1e30 and compare)
 //   2. e = expf(l - max) into LDS (expf_ref: the reference's libm expf, bit
-//      for bit); thread 0 adds them left to right
+//      for bit); chain_sum_block gives their left-to-right sum
 //      (attention.cpp:422-426); p = e * (1/sum)
 //   3. stable sort of the 32-bit keys less the smallest one: order p
 //      descending, ties older first, by sort_buckets; where that declines, up
-//      to 2 kSelThreads tokens sort_small_merge (bitonic within waves, merges in LDS); above: an LSD
-//      radix sort, 4 bits a pass, in registers, skipping digits every key
-//      shares
-//   4. quad sums ((p0+p1)+p2)+p3 of the sorted order in parallel; thread 0
-//      runs the mass loop over them, then the single tokens
+//      to 2 kSelThreads tokens sort_small_merge (bitonic within waves, merges
+//      in LDS); above: an LSD radix sort, 4 bits a pass, in registers, skipping
+//      digits every key shares
+//   4. quad sums ((p0+p1)+p2)+p3 of the sorted order in parallel; the mass loop
+//      over them by chain_sum_block, then the single tokens by thread 0
 //      (attention.cpp:454-472)
 //   5. per-token weights (p * vscale) * isp for the selected tokens, else 0,
 //      written over the logits in token order
@@ -1722,10 +1722,11 @@ __device__ __forceinline__ int vcode_shift(int c) {
 
 // EM: the most tokens a thread (2: up to 2,048 tokens, 4: kFusedMax); OCC: the
 // least blocks a CU that the registers allow.  With the logits given, the
-// selection and the V sum take under 64 registers, so two blocks share a CU:
-// above 256 items, where a second round of blocks would follow, padded 64 runs
-// the logits kernel first too (336 heads d64 K4/V2 x 2,048 tokens: 46 us so, 59
-// in one kernel of 102 registers a block; 672 x 1,024: 55 and 68 us).
+// selection and the V sum take under 64 registers a lane (at 4 tokens a thread
+// 76 to 80 are spilled), so two blocks share a CU: above 256 items,
+// where a second round of blocks would follow, padded 64 runs the logits kernel
+// first too (336 heads d64 K4/V2 x 2,048 tokens: 45 us so, 59 in one kernel of
+// 102 registers a lane; 672 x 1,024: 55 and 68 us).
 template <int PT, int KB, int VB, bool LOGITS_IN, int EM, int OCC>
 __global__ __launch_bounds__(kSelThreads, 4 * OCC) void sparse_fused_kernel(
     HeadDesc *const *item_desc, const float *__restrict__ queries, float v_mass, float inv_sqrt_p,
@@ -1733,7 +1734,7 @@ __global__ __launch_bounds__(kSelThreads, 4 * OCC) void sparse_fused_kernel(
   // one LDS object with the codebooks and the query first: their addresses
   // stay below the 64 KB of a ds_read's immediate offset, so a codebook
   // lookup is one read of the code's byte offset (a separate variable may be
-  // placed after the ~100 KB of SelectShared and cost an add per lookup)
+  // placed after the 55-79 KB of the selection and cost an add per lookup)
   // V pair table (2-bit codes): a nibble of a row, two adjacent codes, to
   // their two centres in one read (16 entries: no bank conflicts; a 256-entry
   // byte table for 4-bit codes conflicts and is slower)

@@ -7,7 +7,7 @@ vscale_t) / sqrt(p) for selected tokens, 0 otherwise, in ring order) are
 compared with the oracle's, token by token: the selected set must be the same,
 and the weights the same bits.  The cases cover every selection code path:
 the fused one-block kernel (rings up to 3,072 tokens at padded 64/128), the
-in-LDS radix sort of the select kernel (up to 8,192 tokens), the per-item
+in-LDS sort of the select kernel (up to 8,192 tokens), the per-item
 multi-block radix sort plus cut kernel above that (up to 65,536 tokens: a
 wrapped 32,768-token ring, exact ties across sort blocks, every probability
 equal) and, above it, the same sort with superblock sums (a plain and a
